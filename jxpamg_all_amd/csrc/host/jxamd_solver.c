@@ -1047,6 +1047,71 @@ static int csr_transpose(int n, int m, const int *ia, const int *ja, const doubl
     return 0;
 }
 
+/* The entries of every row in ascending column order (stable), the first
+ * `keep` of each row left in front.  The hierarchy's coarse rows come in the
+ * order the Galerkin product first touched their columns; sorted, neighbouring
+ * lanes of a row group gather x from the same cache lines (60x220x85: 105-entry
+ * rows 27.2 -> 25.0 us per FP16 polynomial step, the mixed CPR application
+ * 501 -> 484 us). */
+static int csr_sorted(int n, const int *ia, const int *ja, const double *a, int keep, int **oj, double **oa)
+{
+    const size_t nnz = (size_t)ia[n];
+    int *j2 = (int *)malloc(sizeof(int) * (nnz ? nnz : 1));
+    double *a2 = (double *)malloc(sizeof(double) * (nnz ? nnz : 1));
+    if (!j2 || !a2) { free(j2); free(a2); return JXAMD_ERROR_MEMORY; }
+    int bad = 0;
+#pragma omp parallel for schedule(static) reduction(| : bad) if (nnz > 100000)
+    for (int b0 = 0; b0 < n; b0 += 1024) {
+        int cap = 0;
+        int *tj = NULL;
+        double *ta = NULL;
+        for (int i = b0; i < n && i < b0 + 1024; i++) {
+            const int k0 = ia[i], len = ia[i + 1] - k0, f = keep < len ? keep : len, m = len - f;
+            memcpy(j2 + k0, ja + k0, sizeof(int) * (size_t)len);
+            memcpy(a2 + k0, a + k0, sizeof(double) * (size_t)len);
+            int *rj = j2 + k0 + f;
+            double *ra = a2 + k0 + f;
+            if (m > cap) {
+                cap = 2 * m;
+                free(tj);
+                free(ta);
+                tj = (int *)malloc(sizeof(int) * (size_t)cap);
+                ta = (double *)malloc(sizeof(double) * (size_t)cap);
+                if (!tj || !ta) { bad = 1; break; }
+            }
+            /* runs of eight by insertion, then merges */
+            for (int r0 = 0; r0 < m; r0 += 8)
+                for (int x = r0 + 1; x < m && x < r0 + 8; x++) {
+                    const int vj = rj[x];
+                    const double va = ra[x];
+                    int y = x - 1;
+                    for (; y >= r0 && rj[y] > vj; y--) { rj[y + 1] = rj[y]; ra[y + 1] = ra[y]; }
+                    rj[y + 1] = vj;
+                    ra[y + 1] = va;
+                }
+            for (int w = 8; w < m; w *= 2) {
+                for (int lo = 0; lo < m; lo += 2 * w) {
+                    const int mid = lo + w < m ? lo + w : m, hi = lo + 2 * w < m ? lo + 2 * w : m;
+                    int x = lo, y = mid;
+                    for (int o = lo; o < hi; o++) {
+                        const int q = (y >= hi || (x < mid && rj[x] <= rj[y])) ? x++ : y++;
+                        tj[o] = rj[q];
+                        ta[o] = ra[q];
+                    }
+                }
+                memcpy(rj, tj, sizeof(int) * (size_t)m);
+                memcpy(ra, ta, sizeof(double) * (size_t)m);
+            }
+        }
+        free(tj);
+        free(ta);
+    }
+    if (bad) { free(j2); free(a2); return JXAMD_ERROR_MEMORY; }
+    *oj = j2;
+    *oa = a2;
+    return 0;
+}
+
 static int check_csr(const jxamd_csr *c, int square)
 {
     if (!c->ia || !c->ja || !c->a || c->n < 0 || c->ncols < 0) return JXAMD_ERROR_ARG;
@@ -1623,9 +1688,8 @@ static int build_poly(jxamd_solver *s, int l, const jxamd_hierarchy *H)
     return e;
 }
 
-static int build_level(jxamd_solver *s, int l, const jxamd_hierarchy *H)
+static int build_level_mats(jxamd_solver *s, int l, const jxamd_hierarchy *H, const jxamd_csr *A)
 {
-    const jxamd_csr *A = &H->A[l];
     const int n = A->n;
     hsell h;
     int e;
@@ -1734,6 +1798,26 @@ static int build_level(jxamd_solver *s, int l, const jxamd_hierarchy *H)
             (dir > 0 ? &s->Gf[l] : &s->Gb[l])->abytes = level_bytes(dir > 0 ? &s->Gf[l] : &s->Gb[l], A->ia[n], n, 3.0);
         }
     }
+    return 0;
+}
+
+static int build_level(jxamd_solver *s, int l, const jxamd_hierarchy *H)
+{
+    /* the level's matrix with sorted rows (the diagonal still first) where
+     * row groups read it; the one-lane-per-row layouts keep the given order */
+    const jxamd_csr *A = &H->A[l];
+    jxamd_csr S = *A;
+    int *sj = NULL;
+    double *sa = NULL;
+    if (choose_group(A->ia[A->n], A->n) > 1) {
+        CK(csr_sorted(A->n, A->ia, A->ja, A->a, 1, &sj, &sa));
+        S.ja = sj;
+        S.a = sa;
+    }
+    const int e = build_level_mats(s, l, H, &S);
+    free(sj);
+    free(sa);
+    CK(e);
     return build_transfer(s, l, H);
 }
 
