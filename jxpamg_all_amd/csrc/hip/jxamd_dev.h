@@ -70,6 +70,35 @@ int jxamd_k_gs_sweep_grp(int G, int vt, int xt, int nsl, const int *perm, const 
                          const void *val, const float *rsc, const void *diag, const void *f, int fs, const void *uo,
                          void *un, const int *dep_ptr, const int *dep_list, int *sflag, int epoch, int dir,
                          unsigned long long *ticket, unsigned long long *base, int *err, void *stream);
+/* Exact relax-6 sweeps of a small level in one workgroup, the vector in LDS
+ * (k_gs_lds).  A direction's schedule is a list of steps; in step t wavefront
+ * w of `waves` works on a record: 64/G rows of one dependency level, G lanes
+ * per row, U entries per lane (padding: value 0, column n).  Rows of more than
+ * G * U entries take several records in consecutive steps.  Place t * waves + w
+ * of the schedule names the rows and the record (record 0, all padding, where
+ * a wavefront has nothing to do).  JXAMD_LDS_AHEAD steps of padding follow the
+ * last.  Entries lie in 16-byte
+ * vectors: entry u of a lane is component u % E of vector u / E, E = 16 /
+ * sizeof(value) for the values, 4 for the columns, which are byte offsets
+ * into the vector. */
+#define JXAMD_LDS_NONE 0xffffff  /* row number of padding */
+#define JXAMD_LDS_LAST 0x1000000 /* the rows' last record: the new values are formed */
+#define JXAMD_LDS_CONT 0x2000000 /* the rows' sums go on from the previous record */
+#define JXAMD_LDS_AHEAD 4
+typedef struct {
+    const int *row;            /* pairs (place * 64/G + r): row with the flags (the same in every r), record */
+    const unsigned int *col;   /* vector h of lane: (rec * U/4 + h) * 64 + lane */
+    const void *val;           /* vector h of lane: (rec * U/E + h) * 64 + lane */
+    const void *diag;          /* a_ii and 1 / a_ii: diag[2 (rec * 64/G + r)] (a_ii = 0: the row keeps its value) */
+    int steps;                 /* a multiple of three */
+} jxamd_lds_sweep;
+/* rows of vector type xt that fit the device's LDS (0: not available); a
+ * device layer without these two leaves them undefined, and the solver then
+ * keeps to jxamd_k_gs_sweep */
+int jxamd_gs_lds_rows(int xt) __attribute__((weak));
+/* ncalls relax-6 calls (forward, then backward sweep) from uo (NULL: zeros) into un */
+int jxamd_k_gs_lds(int G, int U, int waves, int xt, int n, const jxamd_lds_sweep *fw, const jxamd_lds_sweep *bw,
+                   int ncalls, const void *f, int fs, const void *uo, void *un, void *stream) __attribute__((weak));
 /* stage 2: x^(-1) into slice order, then K fused sweeps (columns of the
  * layout are positions, ~pos for lower neighbours; xs holds K slice-ordered
  * vectors of xstride doubles; the last sweep also writes xout in row order) */

@@ -507,6 +507,145 @@ __global__ void __launch_bounds__(256) k_gs_sweep(int nsl, const int *__restrict
     }
 }
 
+// v of the lane DPP control C selects (row-local, every lane valid)
+template <int C> __device__ __forceinline__ double dpp_mov(double v)
+{
+    const int2 p = __builtin_bit_cast(int2, v);
+    int2 q;
+    q.x = __builtin_amdgcn_update_dpp(0, p.x, C, 0xf, 0xf, true);
+    q.y = __builtin_amdgcn_update_dpp(0, p.y, C, 0xf, 0xf, true);
+    return __builtin_bit_cast(double, q);
+}
+template <int C> __device__ __forceinline__ float dpp_mov(float v)
+{
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), C, 0xf, 0xf, true));
+}
+// sum over aligned groups of G <= 16 lanes, in every lane: quad permutes,
+// then the mirror of a half row and of a row (the quads, then the halves,
+// already hold equal sums), without the LDS round trips of __shfl_xor
+template <int G, typename X> __device__ __forceinline__ X dpp_sum(X v)
+{
+    if (G >= 2) v += dpp_mov<0xB1>(v);  // quad_perm [1,0,3,2]
+    if (G >= 4) v += dpp_mov<0x4E>(v);  // quad_perm [2,3,0,1]
+    if (G >= 8) v += dpp_mov<0x141>(v); // row_half_mirror
+    if (G >= 16) v += dpp_mov<0x140>(v); // row_mirror
+    return v;
+}
+
+// Exact relax-6 sweeps of a level whose vector fits in LDS: one workgroup,
+// the vector updated in place (the host has checked that a row's couplings
+// all lie on other dependency levels: the earlier ones hold new values, the
+// later ones still their old ones).  A dependency level is one step, or a few, and
+// costs a workgroup barrier, LDS gathers, a division and an LDS store, where
+// k_gs_sweep pays a flag round trip through the device's coherence point
+// (about 3 us).  The steps' records do not depend on x: a wavefront holds
+// three in registers, refilled as they are used, so that the loads of a step
+// are issued three steps ahead.
+// Only LDS is ordered at a step's end: the loads stay in flight across it.
+// All sweeps of a level visit run in one launch.  Per sweep, with k_gs_sweep
+// before: 20160 rows of 7 (83 levels) 60 us, 253 before; 8807 rows of 23 (261
+// levels) 153 and 835; 2114 rows of 61 (374 levels) 115 and 1130; 2048 rows
+// of 7 (38 levels) 12 and 102.
+// A step's time is its wavefronts' instructions as much as its latencies
+// (0.35 us with 8-byte loads, packed columns and the compiler's division at
+// G 16, U 8, two wavefronts), hence 16-byte loads at scalar base + lane offset,
+// columns as LDS byte offsets, and the quotient from the stored reciprocal.
+#define LDS_P 3
+
+// a / d with rd = 1 / d rounded: one correction by the exact remainder makes
+// the product the rounded quotient (but for underflow); a remainder that is not finite (a or
+// the quotient infinite or NaN, or 1 / d overflowed) takes the division
+template <typename X> __device__ __forceinline__ X div_by(X a, X d, X rd)
+{
+    const X q = a * rd;
+    const X r = fma(-d, q, a);
+    if (__builtin_expect(!(fabs(r) < (X)__builtin_huge_val()), 0)) return a / d;
+    return fma(r, rd, q);
+}
+
+template <int G, int U, typename X>
+__global__ void __launch_bounds__(1024) k_gs_lds(int n, jxamd_lds_sweep fw, jxamd_lds_sweep bw, int npass, const X *f,
+                                                 int fs, const X *uo, X *un)
+{
+    constexpr int R = WAVE / G;
+    typedef typename vec16<X>::T XV;
+    typedef unsigned int __attribute__((ext_vector_type(4))) UV;
+    typedef X __attribute__((ext_vector_type(2))) X2;
+    constexpr int E = 16 / sizeof(X), NV = U / E, NC = U / 4;
+    extern __shared__ __align__(16) unsigned char smraw[];
+    X *x = reinterpret_cast<X *>(smraw);
+    for (int i = threadIdx.x; i < n; i += blockDim.x) x[i] = uo ? uo[i] : (X)0;
+    if (threadIdx.x == 0) x[n] = 0; // the column of padding entries
+    __syncthreads();
+    const unsigned lane = threadIdx.x % WAVE, gl = lane % G, r = lane / G;
+    const int W = blockDim.x / WAVE, w = wave_id();
+    for (int pass = 0; pass < npass; pass++) {
+        const jxamd_lds_sweep sw = pass & 1 ? bw : fw;
+        int row[LDS_P]; // of the records in registers
+        int2 ra;        // rows and record of the next refill
+        X2 d[LDS_P];
+        X ff[LDS_P];
+        XV v[LDS_P][NV];
+        UV c[LDS_P][NC];
+        auto row_of = [&](int t) {
+            return *(const int2 *)((const char *)sw.row + ((size_t)t * W + w) * (R * sizeof(int2)) + r * sizeof(int2));
+        };
+        auto fill = [&](int p) {
+            const size_t rec = (size_t)__builtin_amdgcn_readfirstlane(ra.y);
+            row[p] = ra.x;
+            ff[p] = *(const X *)((const char *)f + __umul24(min(ra.x & JXAMD_LDS_NONE, n - 1), fs * (int)sizeof(X)));
+            d[p] = *(const X2 *)((const char *)sw.diag + rec * R * sizeof(X2) + r * sizeof(X2));
+            const char *cb = (const char *)sw.col + rec * (NC * WAVE * sizeof(UV));
+            const char *vb = (const char *)sw.val + rec * (NV * WAVE * sizeof(XV));
+#pragma unroll
+            for (int h = 0; h < NC; h++) c[p][h] = *(const UV *)(cb + lane * sizeof(UV) + h * (WAVE * sizeof(UV)));
+#pragma unroll
+            for (int h = 0; h < NV; h++) v[p][h] = *(const XV *)(vb + lane * sizeof(XV) + h * (WAVE * sizeof(XV)));
+        };
+#pragma unroll
+        for (int p = 0; p < LDS_P; p++) {
+            ra = row_of(p);
+            fill(p);
+        }
+        ra = row_of(LDS_P);
+        __builtin_amdgcn_s_waitcnt(0); // the loop's waits then count only its own loads
+        X acc = 0;
+        for (int t = 0; t < sw.steps; t += LDS_P) {
+#pragma unroll
+            for (int p = 0; p < LDS_P; p++) {
+                // loads return in order: the row number of the next refill
+                // goes before this step's record, so that waiting for it
+                // leaves the record's loads in flight
+                const int2 rn = row_of(t + p + LDS_P + 1);
+                const int fl = __builtin_amdgcn_readfirstlane(row[p]);
+                if (!(fl & JXAMD_LDS_CONT)) acc = 0;
+                X xv[U];
+#pragma unroll
+                for (int u = 0; u < U; u++) xv[u] = *reinterpret_cast<const X *>(smraw + c[p][u / 4][u % 4]);
+                __builtin_amdgcn_sched_barrier(0); // every gather issued before the first is waited for
+                X acc2 = 0;
+#pragma unroll
+                for (int u = 0; u < U; u += 2) {
+                    acc += v[p][u / E][u % E] * xv[u];
+                    acc2 += v[p][(u + 1) / E][(u + 1) % E] * xv[u + 1];
+                }
+                acc += acc2;
+                if (fl & JXAMD_LDS_LAST) {
+                    const X sum = dpp_sum<G>(acc);
+                    // a row with a zero diagonal keeps its value
+                    const int i = row[p] & JXAMD_LDS_NONE;
+                    if (gl == 0 && i < n && d[p][0] != (X)0) x[i] = div_by(ff[p] - sum, d[p][0], d[p][1]);
+                }
+                fill(p);
+                ra = rn;
+                asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            }
+        }
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < n; i += blockDim.x) un[i] = x[i];
+}
+
 // K forward block hybrid SOR sweeps on the BSR matrix in one launch
 // (par_relax_bsr.c semantics, one rank), sweep k from x^(k-1) to x^(k):
 //   tmp = omega*b_i - sum_{j<i} A_ij x^(k)_j - sum_{j>i} A_ij x^(k-1)_j
@@ -1860,6 +1999,59 @@ int jxamd_k_gs_sweep(int vt, int xt, int nsl, const int *perm, const int *sptr, 
                     (X_ *)un, dep_ptr, dep_list, sflag, epoch, dir, ticket, *base, err)));
     *base += (unsigned long long)nsl + (unsigned long long)grid * 4;
     return chk(hipGetLastError());
+}
+
+int jxamd_gs_lds_rows(int xt)
+{
+    int dev = 0, lds = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess)
+        return 0;
+    const size_t xsz = xt == JXAMD_T_F64 ? sizeof(double) : sizeof(float);
+    const long rows = (long)(lds / xsz) - 1; // and the padding column
+    return (int)(rows > 65535 ? 65535 : (rows < 0 ? 0 : rows)); // row * fs * size is a 24-bit product
+}
+
+int jxamd_k_gs_lds(int G, int U, int waves, int xt, int n, const jxamd_lds_sweep *fw, const jxamd_lds_sweep *bw,
+                   int ncalls, const void *f, int fs, const void *uo, void *un, void *stream)
+{
+    if (n < 1 || ncalls < 1) return 0;
+    if (waves < 1 || waves > 16 || n > jxamd_gs_lds_rows(xt) || fs < 1 || fs > 1024) return JXAMD_ERROR_ARG;
+    if (fw->steps % LDS_P || bw->steps % LDS_P) return JXAMD_ERROR_ARG;
+    const size_t lds = ((size_t)n + 1) * (xt == JXAMD_T_F64 ? sizeof(double) : sizeof(float));
+    hipStream_t st = (hipStream_t)stream;
+#define LAUNCH_GL(GG, UU, XX)                                                                                          \
+    do {                                                                                                               \
+        const hipError_t e_ = hipFuncSetAttribute((const void *)k_gs_lds<GG, UU, XX>,                                  \
+                                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);               \
+        if (e_ != hipSuccess) return JXAMD_ERROR_DEVICE;                                                               \
+        k_gs_lds<GG, UU, XX><<<1, waves * WAVE, lds, st>>>(n, *fw, *bw, 2 * ncalls, (const XX *)f, fs, (const XX *)uo, \
+                                                           (XX *)un);                                                  \
+        return chk(hipGetLastError());                                                                                 \
+    } while (0)
+#define LAUNCH_GX(GG, UU)                                                                                              \
+    do {                                                                                                               \
+        if (xt == JXAMD_T_F64) LAUNCH_GL(GG, UU, double);                                                             \
+        else LAUNCH_GL(GG, UU, float);                                                                                 \
+    } while (0)
+#define LAUNCH_GU(GG)                                                                                                  \
+    do {                                                                                                               \
+        if (U == 4) LAUNCH_GX(GG, 4);                                                                                  \
+        else if (U == 8) LAUNCH_GX(GG, 8);                                                                             \
+        else return JXAMD_ERROR_ARG;                                                                                   \
+    } while (0)
+    switch (G) {
+    case 1: LAUNCH_GU(1); break;
+    case 2: LAUNCH_GU(2); break;
+    case 4: LAUNCH_GU(4); break;
+    case 8: LAUNCH_GU(8); break;
+    case 16: LAUNCH_GU(16); break;
+    default: return JXAMD_ERROR_ARG;
+    }
+#undef LAUNCH_GU
+#undef LAUNCH_GX
+#undef LAUNCH_GL
+    return JXAMD_ERROR_ARG;
 }
 
 int jxamd_k_bhgs_gather(int npos, int b, const int *perm, const double *x0, const double *xp, int pidx, double *out,

@@ -76,6 +76,13 @@ typedef struct {
     double bytes;
 } dtri;
 
+/* exact relax-6 sweeps of a small level in one workgroup (jxamd_k_gs_lds); W 0: not used */
+typedef struct {
+    int G, U, W;
+    jxamd_lds_sweep sw[2]; /* forward, backward */
+    double abytes;         /* algorithmic bytes of one sweep */
+} dlds;
+
 /* per-kernel-class device timing (HIP events around each launch) */
 #define PROF_POOL 4096
 typedef struct {
@@ -106,6 +113,7 @@ struct jxamd_solver_s {
     int nlev[JXAMD_MAX_LEVELS];
     dsell Ares[JXAMD_MAX_LEVELS], Gf[JXAMD_MAX_LEVELS], Gb[JXAMD_MAX_LEVELS];
     dsell Gc[JXAMD_MAX_LEVELS]; /* threaded relax-6 layout (chunked mode) */
+    dlds Gl[JXAMD_MAX_LEVELS];  /* exact sweeps with the vector in LDS (Gf, Gb are then not built) */
     int *wstep[JXAMD_MAX_LEVELS];
     int nchunks[JXAMD_MAX_LEVELS]; /* 0: sequential sweeps on this level */
     dsell R[JXAMD_MAX_LEVELS], P[JXAMD_MAX_LEVELS];
@@ -1688,6 +1696,179 @@ static int build_poly(jxamd_solver *s, int l, const jxamd_hierarchy *H)
     return e;
 }
 
+/* Rows by dependency level of one direction (ord, level l at start[l] ..
+ * start[l + 1], longer rows first inside a level) for sweeps that update one
+ * vector in place: beside the dependencies, which lie on earlier levels, every
+ * other coupling of a row must lie on a later one (it does for a symmetric
+ * pattern), or the row would read a value that is already new.  *nlev = 0
+ * where that does not hold. */
+static int lds_levels(const jxamd_csr *A, int dir, int *ord, int **ostart, int *nlev)
+{
+    const int n = A->n;
+    int *lev = (int *)malloc(sizeof(int) * (size_t)n);
+    if (!lev) return JXAMD_ERROR_MEMORY;
+    int nl = 0, maxlen = 0, ok = 1;
+    for (int t = 0; t < n; t++) {
+        const int i = dir > 0 ? t : n - 1 - t;
+        int l = 0;
+        for (int k = A->ia[i]; k < A->ia[i + 1]; k++) {
+            const int j = A->ja[k];
+            if ((dir > 0 ? j < i : j > i) && lev[j] + 1 > l) l = lev[j] + 1;
+        }
+        lev[i] = l;
+        if (l + 1 > nl) nl = l + 1;
+        if (A->ia[i + 1] - A->ia[i] > maxlen) maxlen = A->ia[i + 1] - A->ia[i];
+    }
+    for (int i = 0; i < n && ok; i++)
+        for (int k = A->ia[i]; k < A->ia[i + 1]; k++)
+            if ((dir > 0 ? A->ja[k] > i : A->ja[k] < i) && lev[A->ja[k]] <= lev[i]) ok = 0;
+    *nlev = 0;
+    *ostart = NULL;
+    if (!ok) { free(lev); return 0; }
+    int *start = (int *)calloc((size_t)nl + 1, sizeof(int));
+    int *bylen = (int *)malloc(sizeof(int) * (size_t)n);
+    int *cnt = (int *)calloc((size_t)(maxlen > nl ? maxlen : nl) + 2, sizeof(int));
+    if (!start || !bylen || !cnt) { free(lev); free(start); free(bylen); free(cnt); return JXAMD_ERROR_MEMORY; }
+    for (int i = 0; i < n; i++) cnt[maxlen - (A->ia[i + 1] - A->ia[i]) + 1]++;
+    for (int q = 0; q <= maxlen; q++) cnt[q + 1] += cnt[q];
+    for (int i = 0; i < n; i++) bylen[cnt[maxlen - (A->ia[i + 1] - A->ia[i])]++] = i;
+    for (int i = 0; i < n; i++) start[lev[i] + 1]++;
+    for (int l = 0; l < nl; l++) start[l + 1] += start[l];
+    for (int l = 0; l < nl; l++) cnt[l] = start[l];
+    for (int t = 0; t < n; t++) ord[cnt[lev[bylen[t]]]++] = bylen[t];
+    free(lev);
+    free(bylen);
+    free(cnt);
+    *ostart = start;
+    *nlev = nl;
+    return 0;
+}
+
+/* steps of a schedule: a level's rows in slices of R, W slices at a time, a
+ * slice taking one record (in consecutive steps) per G * U entries of its
+ * longest row */
+static long lds_steps(const jxamd_csr *A, const int *ord, const int *start, int nl, int G, int U, int W, long *nrec)
+{
+    const int R = SELLW / G;
+    long steps = 0, recs = 1;
+    for (int l = 0; l < nl; l++)
+        for (int b = start[l]; b < start[l + 1]; b += R) { /* longest row first */
+            const int len = A->ia[ord[b] + 1] - A->ia[ord[b]] - 1, ns = len > G * U ? (len + G * U - 1) / (G * U) : 1;
+            recs += ns;
+            if ((b - start[l]) / R % W == 0) steps += ns;
+        }
+    *nrec = recs;
+    return steps;
+}
+
+/* the schedule and records of one direction, uploaded */
+static int lds_build(const jxamd_solver *s, const jxamd_csr *A, const int *ord, const int *start, int nl, int G, int U,
+                     int W, jxamd_lds_sweep *o)
+{
+    const int R = SELLW / G, n = A->n, xsz = (int)s->xsz, E = 16 / xsz;
+    long nrec = 0, steps = lds_steps(A, ord, start, nl, G, U, W, &nrec);
+    steps = (steps + 2) / 3 * 3;
+    const size_t recs = (size_t)nrec, places = (size_t)(steps + JXAMD_LDS_AHEAD) * W;
+    int *row = (int *)malloc(sizeof(int) * 2 * places * R);
+    double *diag = (double *)malloc(sizeof(double) * 2 * recs * R);
+    int *col = (int *)malloc(sizeof(int) * recs * U * SELLW);
+    double *val = (double *)calloc(recs * U * SELLW, sizeof(double));
+    int e = !row || !diag || !col || !val ? JXAMD_ERROR_MEMORY : 0;
+    if (!e) {
+        for (size_t q = 0; q < places * R; q++) {
+            row[2 * q] = JXAMD_LDS_NONE;
+            row[2 * q + 1] = 0;
+        }
+        for (size_t q = 0; q < 2 * recs * R; q++) diag[q] = 1.0;
+        for (size_t q = 0; q < recs * U * SELLW; q++) col[q] = n * xsz;
+        size_t t = 0, rec = 1;
+        for (int l = 0; l < nl; l++)
+            for (int b = start[l]; b < start[l + 1]; b += R * W) {
+                int tmax = 1;
+                for (int w = 0; w < W; w++) {
+                    const int b0 = b + w * R;
+                    if (b0 >= start[l + 1]) break;
+                    const int len0 = A->ia[ord[b0] + 1] - A->ia[ord[b0]] - 1;
+                    const int ns = len0 > G * U ? (len0 + G * U - 1) / (G * U) : 1;
+                    if (ns > tmax) tmax = ns;
+                    for (int h = 0; h < ns; h++, rec++) {
+                        const size_t place = (t + h) * W + w;
+                        const int fl = (h > 0 ? JXAMD_LDS_CONT : 0) | (h == ns - 1 ? JXAMD_LDS_LAST : 0);
+                        for (int r = 0; r < R; r++) {
+                            row[2 * (place * R + r)] |= fl;
+                            row[2 * (place * R + r) + 1] = (int)rec;
+                            if (b0 + r >= start[l + 1]) continue;
+                            const int i = ord[b0 + r], k0 = A->ia[i] + 1, len = A->ia[i + 1] - k0;
+                            row[2 * (place * R + r)] = i | fl;
+                            /* the diagonal as the kernel holds it, and its reciprocal */
+                            const double di = s->xt == JXAMD_T_F64 ? A->a[A->ia[i]] : (double)(float)A->a[A->ia[i]];
+                            diag[2 * (rec * R + r)] = di;
+                            diag[2 * (rec * R + r) + 1] = di != 0.0 ? 1.0 / di : 0.0;
+                            /* entry pp of the row: record pp / (G U), slot (pp / G) % U, lane pp % G */
+                            for (int pp = h * G * U; pp < len && pp < (h + 1) * G * U; pp++) {
+                                if (A->ja[k0 + pp] == i) continue;
+                                const int u = (pp / G) % U, lane = r * G + pp % G;
+                                col[((rec * (U / 4) + u / 4) * SELLW + lane) * 4 + u % 4] = A->ja[k0 + pp] * xsz;
+                                val[((rec * (U / E) + u / E) * SELLW + lane) * E + u % E] = A->a[k0 + pp];
+                            }
+                        }
+                    }
+                }
+                t += tmax;
+            }
+    }
+    void *dr = NULL, *dc = NULL, *dv = NULL, *dd = NULL;
+    if (!e) e = upload_ints((int **)&dr, row, 2 * places * R, s->stream);
+    if (!e) e = upload_ints((int **)&dc, col, recs * U * SELLW, s->stream);
+    if (!e) e = upload_real(&dv, val, recs * U * SELLW, s->xt, s->stream);
+    if (!e) e = upload_real(&dd, diag, 2 * recs * R, s->xt, s->stream);
+    const int e2 = jxamd_stream_sync(s->stream);
+    o->row = (const int *)dr;
+    o->col = (const unsigned int *)dc;
+    o->val = dv;
+    o->diag = dd;
+    o->steps = (int)steps;
+    free(row); free(diag); free(col); free(val);
+    return e ? e : e2;
+}
+
+/* Exact sweeps of level l with its vector in LDS, where it fits and where one
+ * workgroup is the faster.  Measured: a step of W wavefronts with U entries
+ * per lane takes 0.2 + 0.0075 U W us (barrier, gathers, division; the
+ * wavefronts' instructions), records beyond the L2 come at some 45 GB/s;
+ * k_gs_sweep takes about 3 us per dependency level on the whole device. */
+static int build_lds(jxamd_solver *s, int l, const jxamd_csr *A)
+{
+    dlds *g = &s->Gl[l];
+    const int n = A->n, cap = jxamd_gs_lds_rows && jxamd_k_gs_lds ? jxamd_gs_lds_rows(s->xt) : 0;
+    if (n < 1 || n > cap || s->vt != s->xt) return 0;
+    int *ord[2] = {NULL, NULL}, *start[2] = {NULL, NULL}, nl[2] = {0, 0}, e = 0;
+    for (int d = 0; d < 2 && !e; d++) {
+        ord[d] = (int *)malloc(sizeof(int) * (size_t)n);
+        e = ord[d] ? lds_levels(A, d ? -1 : 1, ord[d], &start[d], &nl[d]) : JXAMD_ERROR_MEMORY;
+    }
+    if (!e && nl[0] && nl[1]) {
+        double best = 3.0 * nl[0];
+        int G = 0, U = 0, W = 0;
+        for (int g1 = 1; g1 <= 16; g1 *= 2)
+            for (int u1 = 4; u1 <= 8; u1 += 4)
+                for (int w1 = 1; w1 <= 16; w1 *= 2) {
+                    long nrec = 0;
+                    const long steps = lds_steps(A, ord[0], start[0], nl[0], g1, u1, w1, &nrec);
+                    const double bytes = (double)nrec * SELLW * u1 * (4.0 + (double)s->xsz);
+                    const double lane = (0.2 + 0.0075 * u1 * w1) * (double)steps;
+                    const double c = bytes > 2.0e6 && bytes / 45.0e3 > lane ? bytes / 45.0e3 : lane;
+                    if (c < best) { best = c; G = g1; U = u1; W = w1; }
+                }
+        for (int d = 0; d < 2 && !e && W; d++) e = lds_build(s, A, ord[d], start[d], nl[d], G, U, W, &g->sw[d]);
+        g->G = G;
+        g->U = U;
+        g->W = e ? 0 : W;
+    }
+    for (int d = 0; d < 2; d++) { free(ord[d]); free(start[d]); }
+    return e;
+}
+
 static int build_level_mats(jxamd_solver *s, int l, const jxamd_hierarchy *H, const jxamd_csr *A)
 {
     const int n = A->n;
@@ -1713,6 +1894,7 @@ static int build_level_mats(jxamd_solver *s, int l, const jxamd_hierarchy *H, co
     if (s->prm.relax_threads > 1) T = s->prm.relax_threads;
     else if (s->prm.relax_chunk > 0) T = (n + s->prm.relax_chunk - 1) / s->prm.relax_chunk;
     if (T > n) T = n;
+    if (T <= 1 && (l < s->L - 1 || s->L == 1)) CK(build_lds(s, l, A));
     if (T > 1 && (l < s->L - 1 || s->L == 1) && jxamd_gs_chunk_lds_rows(n, T) <= JXAMD_CHUNK_LDS_MAX) {
         /* short chunks: one pass, off-diagonals in natural row order (SELL),
          * or full CSR rows read by row groups */
@@ -1762,6 +1944,10 @@ static int build_level_mats(jxamd_solver *s, int l, const jxamd_hierarchy *H, co
         s->nchunks[l] = T;
         /* forward + backward pass over the matrix, old + new + rhs vectors */
         s->Gc[l].abytes = 2.0 * level_bytes(&s->Gc[l], A->ia[n], n, 0.0) + 3.0 * type_size(s->xt) * n;
+    } else if ((l < s->L - 1 || s->L == 1) && s->Gl[l].W) {
+        /* sweep: matrix once + old x + new x + rhs */
+        dsell t = {.vt = s->vt, .xt = s->xt};
+        s->Gl[l].abytes = level_bytes(&t, A->ia[n], n, 3.0);
     } else if ((l < s->L - 1 || s->L == 1) && GA > 1) {
         /* long rows: sweep orders with slices of 64/GA rows of one dependency
          * level, each row summed by a group of GA lanes over its plain CSR
@@ -1961,6 +2147,11 @@ int jxamd_solver_destroy(jxamd_solver *s)
     jxamd_dev_free(d->val32); jxamd_dev_free(d->dinv32); jxamd_dev_free(d->rsc16); jxamd_dev_free(d->pptr16);
     for (int l = 0; l < JXAMD_MAX_LEVELS; l++) {
         dsell_free(&s->Ares[l]); dsell_free(&s->Gf[l]); dsell_free(&s->Gb[l]); dsell_free(&s->Gc[l]);
+        for (int d = 0; d < 2; d++) {
+            const jxamd_lds_sweep *w = &s->Gl[l].sw[d];
+            jxamd_dev_free((void *)w->row); jxamd_dev_free((void *)w->col);
+            jxamd_dev_free((void *)w->val); jxamd_dev_free((void *)w->diag);
+        }
         jxamd_dev_free(s->wstep[l]);
         jxamd_dev_free(s->dinvl[l]);
         dsell_free(&s->R[l]); dsell_free(&s->P[l]);
@@ -2039,6 +2230,17 @@ static int hsgs(jxamd_solver *s, int l, const void *f, int fs, void *u, int uo_z
                                 &s->tbase, s->err, s->stream));
         prof_end_level(s, pq, JXAMD_PROF_GS_SWEEP, l, g->abytes);
     }
+    return 0;
+}
+
+/* relax-6 calls of a level whose vector is kept in LDS, in one launch */
+static int hsgs_lds(jxamd_solver *s, int l, const void *f, int fs, void *u, int uo_zero, int ncalls)
+{
+    const dlds *g = &s->Gl[l];
+    int pq = prof_begin(s);
+    CK(jxamd_k_gs_lds(g->G, g->U, g->W, s->xt, s->nlev[l], &g->sw[0], &g->sw[1], ncalls, f, fs, uo_zero ? NULL : u, u,
+                      s->stream));
+    prof_end_level(s, pq, JXAMD_PROF_GS_SWEEP, l, 2.0 * ncalls * g->abytes);
     return 0;
 }
 
@@ -2123,6 +2325,7 @@ static int relax_pair(jxamd_solver *s, int l, const void *f, int fs, void *u, in
         CK(hsgs_chunk(s, l, f, fs, uo_zero ? NULL : u, s->T[l]));
         return hsgs_chunk(s, l, f, fs, s->T[l], u);
     }
+    if (s->Gl[l].W) return hsgs_lds(s, l, f, fs, u, uo_zero, 2);
     CK(hsgs(s, l, f, fs, u, uo_zero));
     return hsgs(s, l, f, fs, u, 0);
 }
@@ -2135,6 +2338,7 @@ static int relax_once(jxamd_solver *s, int l, const void *f, int fs, void *u, in
         CK(hsgs_chunk(s, l, f, fs, uo_zero ? NULL : u, s->T[l]));
         return jxamd_d2d(u, s->T[l], s->xsz * s->nlev[l], s->stream);
     }
+    if (s->Gl[l].W) return hsgs_lds(s, l, f, fs, u, uo_zero, 1);
     return hsgs(s, l, f, fs, u, uo_zero);
 }
 
