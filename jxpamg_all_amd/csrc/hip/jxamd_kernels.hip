@@ -12,9 +12,9 @@
 //   positions are sorted by dependency level so a wavefront's rows become
 //   ready together.  The diagonal is kept apart (diag[p]).
 //
-// Sync-free sweeps (k_gs_sweep, k_bhgs_sweep) run persistent wavefronts over
-// level-pure slices with per-slice completion flags; every wait is bounded
-// and an overflow is recorded in err[0] (see the comment at the kernels).
+// Sync-free sweeps (k_gs_sweep, k_bhgs_multi, k_btri) run persistent wavefronts
+// over level-pure slices whose results are their own flags; every wait is
+// bounded and an overflow is recorded in err[0] (see the comment at the kernels).
 #include <hip/hip_fp16.h>
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -424,45 +424,166 @@ __global__ void __launch_bounds__(256) k_poly_step(int n, const int *__restrict_
 // give, per slice, the earlier slices holding its rows' dependencies.  Waves
 // are persistent: each claims slices in order from the ticket counter (so a
 // claimed slice's dependencies belong to slices claimed before it, all held
-// by running waves), loads its row data, waits on its dependency slices'
-// flags (bounded), takes an acquire fence, computes, stores with device-
-// coherent stores and publishes sflag[slice] = epoch with release semantics.
-// Every wave ends with exactly one failed claim, so a launch consumes
-// nsl + (number of waves) tickets.
+// by running waves) and loads all that does not depend on the launch's own
+// results.  Every wave ends with exactly one failed claim, so a launch
+// consumes nsl + (number of waves) tickets.
+//
+// A result is its own flag: the vector a launch fills holds the armed pattern
+// (a signalling NaN, which no arithmetic produces) until a row stores its
+// value, and a dependent row reads the values themselves until none is armed.
+// One dependency level costs one store and one load through the device's
+// coherence point.  With a flag per slice it cost four such trips in a row:
+// the store acknowledged, the flag stored, the flag polled, the values loaded
+// (and the column indices and matrix entries, which now come before the wait).
+// So that the waves of later levels do not flood the memory system with such
+// reads, a wave first polls one word, the flag of a slice two levels earlier;
+// that flag is raised with no ordering and carries no promise.  Waits are
+// bounded: a wave that gives up sets err[0] and goes on with the armed NaN,
+// which arithmetic quiets, so the launch still drains.
+// Measured, with a flag per slice and now: a 3x3 BILU(0) triangle of 30x40x25
+// (93 levels) 261 and 214 us; three stage-2 sweeps of 24x40x21, b = 2, 252 and
+// 134 us, of 16x16x8, b = 3, 126 and 75 us; the reference-exact CPR application
+// of 60x220x85 255 and 89 ms.  A level costs 2.1-2.3 us now.
 // ---------------------------------------------------------------------------
+#define ARMED_F64 0x7ff4a5a5a5a5a5a5ull
+#define ARMED_F32 0x7fa5a5a5u
+__device__ __forceinline__ bool is_armed(double v) { return __builtin_bit_cast(unsigned long long, v) == ARMED_F64; }
+__device__ __forceinline__ bool is_armed(float v) { return __builtin_bit_cast(unsigned int, v) == ARMED_F32; }
+template <typename X> __device__ __forceinline__ X armed_value();
+template <> __device__ __forceinline__ double armed_value() { return __builtin_bit_cast(double, ARMED_F64); }
+template <> __device__ __forceinline__ float armed_value() { return __builtin_bit_cast(float, ARMED_F32); }
+// a value a caller passed in may hold the armed bits; it becomes another NaN
+__device__ __forceinline__ double disarmed(double v)
+{
+    return is_armed(v) ? __builtin_bit_cast(double, ARMED_F64 | (1ull << 51)) : v;
+}
+__device__ __forceinline__ float disarmed(float v)
+{
+    return is_armed(v) ? __builtin_bit_cast(float, ARMED_F32 | (1u << 22)) : v;
+}
+template <typename X> __device__ __forceinline__ void st_result(X *p, X v) { st_coherent(p, disarmed(v)); }
+
+// arms the b values of every row at positions 0..npos-1 (perm == nullptr: of
+// entries 0..npos-1)
+template <typename X>
+__global__ void __launch_bounds__(256) k_arm(long long npos, int b, const int *__restrict__ perm, X *y)
+{
+    const long long p = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (p >= npos) return;
+    const long long i = perm ? perm[p] : p;
+    if (i < 0) return;
+    for (int q = 0; q < b; q++) st_coherent(y + i * b + q, armed_value<X>());
+}
+
 __device__ __forceinline__ int claim_slice(unsigned long long *ticket, unsigned long long base, int lane)
 {
     int s = 0;
     if (lane == 0) s = (int)(__hip_atomic_fetch_add(ticket, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) - base);
-    return __shfl(s, 0);
+    return __builtin_amdgcn_readfirstlane(s);
 }
 
-__device__ __forceinline__ void wait_slices(const int *__restrict__ dep_ptr, const int *__restrict__ dep_list,
-                                            const int *sflag, int s, int epoch, int lane, int *err)
+// latest slice slice s depends on (-1: none)
+__device__ __forceinline__ int latest_dep(const int *__restrict__ dep_ptr, const int *__restrict__ dep_list, int s,
+                                          int lane)
 {
-    const int d0 = dep_ptr[s], d1 = dep_ptr[s + 1];
-    for (int q = d0 + lane; q < d1; q += WAVE) {
-        const int w = dep_list[q];
-        int spins = 0, nap = 0;
-        while (!flag_ready(ld_flag(sflag + w), epoch)) {
-            if (++spins > SPIN_LIMIT) {
-                __hip_atomic_store(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                break;
-            }
-            if (nap < 4) { __builtin_amdgcn_s_sleep(1); nap++; }
-            else __builtin_amdgcn_s_sleep(4);
+    int w = -1;
+    const int d1 = dep_ptr[s + 1];
+    for (int q = dep_ptr[s] + lane; q < d1; q += WAVE) w = max(w, dep_list[q]);
+    for (int o = WAVE / 2; o > 0; o /= 2) w = max(w, __shfl_xor(w, o));
+    return __builtin_amdgcn_readfirstlane(w);
+}
+// the slice whose flag slice s polls before it reads values: the latest its
+// latest dependency depends on (-1: none)
+__device__ __forceinline__ int gate_slice(const int *__restrict__ dep_ptr, const int *__restrict__ dep_list, int s,
+                                          int lane)
+{
+    const int w = latest_dep(dep_ptr, dep_list, s, lane);
+    return w < 0 ? -1 : latest_dep(dep_ptr, dep_list, w, lane);
+}
+__device__ __forceinline__ void wait_gate(const int *sflag, int g, int epoch)
+{
+    if (g < 0) return;
+    for (int spins = 0; !flag_ready(ld_flag(sflag + g), epoch) && spins < SPIN_LIMIT; spins++)
+        __builtin_amdgcn_s_sleep(1);
+}
+__device__ __forceinline__ void raise_gate(int *sflag, int s, int epoch)
+{
+    __hip_atomic_store(sflag + s, epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// v[u][q] = x[b j[u] + q] where use[u] (0 elsewhere), once none is armed
+template <int U, int B, typename X>
+__device__ __forceinline__ void read_results(const X *x, const int (&j)[U], const bool (&use)[U], X (&v)[U][B], int *err)
+{
+    for (int spins = 0;; spins++) {
+        bool wait = false;
+#pragma unroll
+        for (int u = 0; u < U; u++)
+#pragma unroll
+            for (int q = 0; q < B; q++) v[u][q] = use[u] ? ld_coherent(x + (size_t)j[u] * B + q) : (X)0;
+#pragma unroll
+        for (int u = 0; u < U; u++)
+#pragma unroll
+            for (int q = 0; q < B; q++) wait |= is_armed(v[u][q]);
+        if (!wait) break;
+        if (spins >= SPIN_LIMIT) {
+            __hip_atomic_store(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            break;
         }
     }
-    // The flag loads have returned (the loop waited on them); the dependent
-    // data is read afterwards with device-scope atomic loads (see
-    // st_flag_release), so only a compiler barrier is needed here.
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
 }
+
+// U entries of a lane's row for a Gauss-Seidel sweep: entry u is number
+// k + u * G of the row, at index (k + u * G) * ST + off of col and val
+// (SELL-64: ST = 64, off = lane; plain rows: ST = 1, off = 0), for numbers
+// below ke.  A dependency is j < i (dir > 0) or j > i.
+template <int U, int G, int ST, typename V, typename X> struct gs_batch {
+    int j[U];
+    V v[U];
+    __device__ __forceinline__ void load(int k, int ke, int off, const int *__restrict__ col, const V *__restrict__ val)
+    {
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const size_t e = (size_t)(k + u * G) * ST + off;
+            const bool in = k + u * G < ke;
+            j[u] = in ? col[e] : -1;
+            v[u] = in ? val[e] : (V)0;
+        }
+    }
+    __device__ __forceinline__ bool coupled(int u, int i, int dir, bool dep) const
+    {
+        return j[u] >= 0 && j[u] != i && (dir > 0 ? j[u] < i : j[u] > i) == dep;
+    }
+    // sum over the couplings that are no dependencies, entry values x
+    __device__ __forceinline__ X others(int i, int dir, const X *x) const
+    {
+        X xv[U], acc = 0;
+#pragma unroll
+        for (int u = 0; u < U; u++) xv[u] = coupled(u, i, dir, false) ? x[j[u]] : (X)0;
+#pragma unroll
+        for (int u = 0; u < U; u++) acc += (X)cvt(v[u]) * xv[u];
+        return acc;
+    }
+    // sum over the dependencies, this launch's values x
+    __device__ __forceinline__ X dependencies(int i, int dir, const X *x, int *err) const
+    {
+        X xv[U][1], acc = 0;
+        bool use[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) use[u] = coupled(u, i, dir, true);
+        read_results<U, 1, X>(x, j, use, xv, err);
+#pragma unroll
+        for (int u = 0; u < U; u++)
+            if (use[u]) acc += (X)cvt(v[u]) * xv[u][0];
+        return acc;
+    }
+};
 
 // One Gauss-Seidel sweep of hybrid SSOR (relax 6, weights 1).
 //   dir > 0: forward (dependencies j < i), dir < 0: backward (j > i).
-//   Old values from uo (zeros if uo == nullptr), new values into un.
+//   Old values from uo (zeros if uo == nullptr), new values into un (armed).
 //   f may be strided (fs).  A row with a zero diagonal keeps its old value.
+// Bound by the dependency levels' round trips (see above); a row's first
+// SELL_U entries stay in registers across the wait.
 template <typename V, typename X>
 __global__ void __launch_bounds__(256) k_gs_sweep(int nsl, const int *__restrict__ perm, const int *__restrict__ sptr,
                                                   const int *__restrict__ col, const V *__restrict__ val,
@@ -478,32 +599,35 @@ __global__ void __launch_bounds__(256) k_gs_sweep(int nsl, const int *__restrict
         if (s < 0 || s >= nsl) break;
         const int p = s * WAVE + lane;
         const int i = perm[p];
-        const int k0 = sptr[s], k1 = sptr[s + 1];
+        const int k0 = sptr[s], k1 = i >= 0 ? sptr[s + 1] : k0;
         X res = 0, d = 1, uold_i = 0, sc = 1;
         if (i >= 0) {
             d = diag[p];
             res = f[(size_t)i * fs];
             if (uo) uold_i = uo[i];
             if (row_scaled<V>::value) sc = (X)rsc[p];
-            // terms on old values need no wait
-            for (int k = k0; k < k1; k++) {
-                const size_t e = (size_t)k * WAVE + lane;
-                const int j = col[e];
-                const bool dep = dir > 0 ? (j < i) : (j > i);
-                if (!dep && j != i && uo) res -= sc * (X)cvt(val[e]) * uo[j];
+        }
+        typedef gs_batch<SELL_U, 1, WAVE, V, X> batch;
+        batch first;
+        first.load(k0, k1, lane, col, val);
+        X acc = 0;
+        if (uo) {
+            acc = first.others(i, dir, uo);
+            for (int k = k0 + SELL_U; k < k1; k += SELL_U) {
+                batch t;
+                t.load(k, k1, lane, col, val);
+                acc += t.others(i, dir, uo);
             }
         }
-        wait_slices(dep_ptr, dep_list, sflag, s, epoch, lane, err);
-        if (i >= 0) {
-            for (int k = k0; k < k1; k++) {
-                const size_t e = (size_t)k * WAVE + lane;
-                const int j = col[e];
-                const bool dep = dir > 0 ? (j < i) : (j > i);
-                if (dep) res -= sc * (X)cvt(val[e]) * ld_coherent(un + j);
-            }
-            st_coherent(un + i, d != (X)0 ? res / d : uold_i);
+        wait_gate(sflag, gate_slice(dep_ptr, dep_list, s, lane), epoch);
+        acc += first.dependencies(i, dir, un, err);
+        for (int k = k0 + SELL_U; k < k1; k += SELL_U) {
+            batch t;
+            t.load(k, k1, lane, col, val);
+            acc += t.dependencies(i, dir, un, err);
         }
-        st_flag_release(sflag + s, epoch);
+        if (i >= 0) st_result(un + i, d != (X)0 ? (res - sc * acc) / d : uold_i);
+        raise_gate(sflag, s, epoch);
     }
 }
 
@@ -537,13 +661,12 @@ template <int G, typename X> __device__ __forceinline__ X dpp_sum(X v)
 // all lie on other dependency levels: the earlier ones hold new values, the
 // later ones still their old ones).  A dependency level is one step, or a few, and
 // costs a workgroup barrier, LDS gathers, a division and an LDS store, where
-// k_gs_sweep pays a flag round trip through the device's coherence point
-// (about 3 us).  The steps' records do not depend on x: a wavefront holds
+// k_gs_sweep pays a round trip through the device's coherence point (2 us).  The steps' records do not depend on x: a wavefront holds
 // three in registers, refilled as they are used, so that the loads of a step
 // are issued three steps ahead.
 // Only LDS is ordered at a step's end: the loads stay in flight across it.
-// All sweeps of a level visit run in one launch.  Per sweep, with k_gs_sweep
-// before: 20160 rows of 7 (83 levels) 60 us, 253 before; 8807 rows of 23 (261
+// All sweeps of a level visit run in one launch.  Per sweep, with a flag-per-slice
+// k_gs_sweep before: 20160 rows of 7 (83 levels) 60 us, 253 before; 8807 rows of 23 (261
 // levels) 153 and 835; 2114 rows of 61 (374 levels) 115 and 1130; 2048 rows
 // of 7 (38 levels) 12 and 102.
 // A step's time is its wavefronts' instructions as much as its latencies
@@ -652,11 +775,8 @@ __global__ void __launch_bounds__(1024) k_gs_lds(int n, jxamd_lds_sweep fw, jxam
 //         + (1-omega) sum_{j!=i} A_ij x^(k-1)_j
 //   x^(k)_i = (1 - w*omega) x^(k-1)_i + w * Dinv_i tmp
 // Every x^(k) lives in slice order: the B values of the row at position p
-// (perm[p] = i) sit at xs + k*xstride + p*B; x^(-1) is xsl0 in the same
-// order.  A slice's 64 rows fill exactly 12 (B = 3) or 8/16 (B = 2/4) whole
-// 128-byte lines, so a line is read only after the flag of the one slice that
-// writes it: ordinary cached loads then see final values, and only the
-// stores (written through at device scope) and the flags need coherence.
+// (perm[p] = i) sit at xs + k*xstride + p*B, armed when the launch starts;
+// x^(-1) is xsl0 in the same order.
 // Columns of the layout are positions, bit-inverted (~pos) for lower
 // neighbours (j < i); the final sweep also stores x in row order into xout.
 // Work items are virtual slices v = k*nsl + s taken in the order vorder (the
@@ -665,15 +785,16 @@ __global__ void __launch_bounds__(1024) k_gs_lds(int n, jxamd_lds_sweep fw, jxam
 //   (k, s) after (k-1, s'') for s'' in dall(s) (slices of all neighbours, s)
 // so sweep k+1 starts on a slice as soon as sweep k has passed its
 // neighbourhood: the K sweeps overlap instead of running back to back.
-// Flags: sflag[k*nsl + s].
-template <int B>
+// Gate flags: sflag[k*nsl + s].  U slots per batch: the stencil's six for
+// B <= 3 (their blocks stay in registers from before the first wait), half
+// of them for B = 4, whose blocks fill the registers.
+template <int B, int U>
 __global__ void __launch_bounds__(256)
 k_bhgs_multi(int nsl, int nvs, const int *__restrict__ vorder, const int *__restrict__ perm,
              const int *__restrict__ sptr, const int *__restrict__ col, const double *__restrict__ val,
              const double *__restrict__ dinv, const double *__restrict__ rhs, const double *__restrict__ xsl0,
              double *xs, long long xstride, double *__restrict__ xout, const int *__restrict__ dlo_ptr,
-             const int *__restrict__ dlo_list, const int *__restrict__ dall_ptr, const int *__restrict__ dall_list,
-             int *sflag, int epoch, double w, double omega, unsigned long long *ticket, unsigned long long base,
+             const int *__restrict__ dlo_list, int *sflag, int epoch, double w, double omega, unsigned long long *ticket, unsigned long long base,
              int *err)
 {
     const int lane = threadIdx.x % WAVE;
@@ -685,62 +806,78 @@ k_bhgs_multi(int nsl, int nvs, const int *__restrict__ vorder, const int *__rest
         const int k = v / nsl, s = v - k * nsl;
         double *xn = xs + (size_t)k * xstride;
         const double *xo = k == 0 ? xsl0 : xs + (size_t)(k - 1) * xstride;
-        if (k > 0) wait_slices(dall_ptr, dall_list, sflag + (size_t)(k - 1) * nsl, s, epoch, lane, err);
         const int p = s * WAVE + lane;
         const int i = perm[p];
-        const int k0 = sptr[s], k1 = sptr[s + 1];
-        double res0[B], res2[B];
+        const int k0 = sptr[s], k1 = i >= 0 ? sptr[s + 1] : k0;
+        double res0[B], res2[B], rb[B], D[B * B];
 #pragma unroll
-        for (int r = 0; r < B; r++) { res0[r] = 0.0; res2[r] = 0.0; }
-        if (i >= 0) {
+        for (int r = 0; r < B; r++) {
+            res0[r] = 0.0;
+            res2[r] = 0.0;
+            rb[r] = i >= 0 ? rhs[(size_t)i * B + r] : 0.0;
+        }
+#pragma unroll
+        for (int q = 0; q < B * B; q++) D[q] = i >= 0 ? dinv[(size_t)i * B * B + q] : 0.0;
+        const int gate = gate_slice(dlo_ptr, dlo_list, s, lane);
+        int *flag = sflag + (size_t)k * nsl;
+        bool gated = false;
+        for (int kk = k0; kk < k1; kk += U) {
+            int jp[U];
+            bool use[U], lower[U];
+            double a[U][B * B], x[U][B];
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const int c = kk + u < k1 ? col[(size_t)(kk + u) * WAVE + lane] : p;
+                lower[u] = c < 0;
+                jp[u] = lower[u] ? ~c : c;
+                use[u] = jp[u] != p; // the row's own position pads
+            }
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const double *vv = val + (size_t)(use[u] ? kk + u : k0) * B * B * WAVE + lane;
+#pragma unroll
+                for (int e = 0; e < B * B; e++) a[u][e] = vv[e * WAVE];
+            }
+            if (!gated) wait_gate(flag, gate, epoch);
+            gated = true;
             // all old-value terms, and the current-value terms of upper neighbours
-            for (int kk = k0; kk < k1; kk++) {
-                const int c = col[(size_t)kk * WAVE + lane];
-                const bool lower = c < 0;
-                const int jp = lower ? ~c : c;
-                if (jp == p) continue; // padding slot
-                double xold[B];
+            if (k > 0) {
+                read_results<U, B, double>(xo, jp, use, x, err);
+            } else {
 #pragma unroll
-                for (int q = 0; q < B; q++) xold[q] = xo[(size_t)jp * B + q];
-                const double *vv = val + (size_t)kk * B * B * WAVE + lane;
+                for (int u = 0; u < U; u++)
 #pragma unroll
-                for (int r = 0; r < B; r++) {
-#pragma unroll
-                    for (int q = 0; q < B; q++) {
-                        const double a = vv[(r * B + q) * WAVE];
-                        res2[r] += a * xold[q];
-                        if (!lower) res0[r] -= a * xold[q];
-                    }
-                }
+                    for (int q = 0; q < B; q++) x[u][q] = use[u] ? xo[(size_t)jp[u] * B + q] : 0.0;
             }
+#pragma unroll
+            for (int u = 0; u < U; u++)
+                if (use[u])
+#pragma unroll
+                    for (int r = 0; r < B; r++)
+#pragma unroll
+                        for (int q = 0; q < B; q++) {
+                            res2[r] += a[u][r * B + q] * x[u][q];
+                            if (!lower[u]) res0[r] -= a[u][r * B + q] * x[u][q];
+                        }
+            read_results<U, B, double>(xn, jp, lower, x, err);
+#pragma unroll
+            for (int u = 0; u < U; u++)
+                if (lower[u])
+#pragma unroll
+                    for (int r = 0; r < B; r++)
+#pragma unroll
+                        for (int q = 0; q < B; q++) res0[r] -= a[u][r * B + q] * x[u][q];
         }
-        double xi[B], rb[B], D[B * B];
         if (i >= 0) {
+            const int self[1] = {p};
+            const bool one[1] = {true};
+            double xi[1][B], tmp[B];
+            if (k > 0) {
+                read_results<1, B, double>(xo, self, one, xi, err);
+            } else {
 #pragma unroll
-            for (int r = 0; r < B; r++) {
-                xi[r] = xo[(size_t)p * B + r];
-                rb[r] = rhs[(size_t)i * B + r];
+                for (int q = 0; q < B; q++) xi[0][q] = xo[(size_t)p * B + q];
             }
-#pragma unroll
-            for (int q = 0; q < B * B; q++) D[q] = dinv[(size_t)i * B * B + q];
-        }
-        wait_slices(dlo_ptr, dlo_list, sflag + (size_t)k * nsl, s, epoch, lane, err);
-        if (i >= 0) {
-            for (int kk = k0; kk < k1; kk++) {
-                const int c = col[(size_t)kk * WAVE + lane];
-                if (c >= 0) continue;
-                const int jp = ~c;
-                double xc[B];
-#pragma unroll
-                for (int q = 0; q < B; q++) xc[q] = xn[(size_t)jp * B + q];
-                const double *vv = val + (size_t)kk * B * B * WAVE + lane;
-#pragma unroll
-                for (int r = 0; r < B; r++) {
-#pragma unroll
-                    for (int q = 0; q < B; q++) res0[r] -= vv[(r * B + q) * WAVE] * xc[q];
-                }
-            }
-            double tmp[B];
 #pragma unroll
             for (int r = 0; r < B; r++) tmp[r] = omega * rb[r] + res0[r] + (1.0 - omega) * res2[r];
             const double prod = 1.0 - w * omega;
@@ -749,12 +886,12 @@ k_bhgs_multi(int nsl, int nvs, const int *__restrict__ vorder, const int *__rest
                 double o = 0.0;
 #pragma unroll
                 for (int q = 0; q < B; q++) o += D[r * B + q] * tmp[q];
-                const double xv = xi[r] * prod + w * o;
-                st_coherent(xn + (size_t)p * B + r, xv);
+                const double xv = xi[0][r] * prod + w * o;
+                st_result(xn + (size_t)p * B + r, xv);
                 if (k == K - 1) xout[(size_t)i * B + r] = xv;
             }
         }
-        st_flag_release(sflag + (size_t)k * nsl + s, epoch);
+        raise_gate(flag, s, epoch);
     }
 }
 
@@ -963,10 +1100,10 @@ __global__ void k_bhgs_gather(int npos, int B, const int *__restrict__ perm, con
 // backward U solve), stored as V (double, float, or __half scaled by the
 // power of two rsc[p] per block row: M_ij = rsc[p] * stored; FP16 elements
 // stored in pairs, slot k's word w at (k * ceil(B*B/2) + w) * 64 + lane), Dinv as DV,
-// vectors and arithmetic double.  A lane loads the column indices of BT_U
-// blocks, then their values and the dependency values, before it uses any,
-// so one level step costs two dependent round trips rather than two per
-// block.  The subtractions keep the order of the blocks in the row.
+// vectors and arithmetic double.  A lane loads the column indices and blocks
+// of its first BT_U slots before it waits, so that a level step costs the
+// dependency values' round trip and no more (out is armed when the launch
+// starts).  The subtractions keep the order of the blocks in the row.
 #define BT_U 4
 template <int B, typename V, typename DV>
 __global__ void __launch_bounds__(256) k_btri(int nsl, const int *__restrict__ perm, const int *__restrict__ sptr,
@@ -994,61 +1131,64 @@ __global__ void __launch_bounds__(256) k_btri(int nsl, const int *__restrict__ p
             }
             if (rsc) sc = (double)rsc[p];
         }
-        wait_slices(dep_ptr, dep_list, sflag, s, epoch, lane, err);
-        if (i >= 0) {
-            for (int k = k0; k < k1; k += BT_U) {
-                int j[BT_U];
+        const int gate = gate_slice(dep_ptr, dep_list, s, lane);
+        for (int k = k0; k < k1; k += BT_U) {
+            int j[BT_U];
+            bool use[BT_U];
+            double xc[BT_U][B], m[BT_U][B * B];
 #pragma unroll
-                for (int u = 0; u < BT_U; u++) j[u] = k + u < k1 ? col[(size_t)(k + u) * WAVE + lane] : i;
-                double xc[BT_U][B];
-                double m[BT_U][B * B];
+            for (int u = 0; u < BT_U; u++) {
+                j[u] = k + u < k1 && i >= 0 ? col[(size_t)(k + u) * WAVE + lane] : i;
+                use[u] = j[u] != i; // the row itself marks a padding slot (and the batch's tail)
+            }
 #pragma unroll
-                for (int u = 0; u < BT_U; u++) {
-                    // the row itself marks a padding slot (and the batch's tail)
+            for (int u = 0; u < BT_U; u++) {
+                const size_t ks = k + u < k1 ? k + u : k0;
+                if constexpr (constexpr_is_half<V>::value) {
+                    // FP16: elements 2w and 2w + 1 of a block in one
+                    // 32-bit word (a zero high half past the last), so
+                    // the loads are whole words
+                    constexpr int NW = (B * B + 1) / 2;
+                    const __half2 *vw = reinterpret_cast<const __half2 *>(val) + ks * NW * WAVE + lane;
 #pragma unroll
-                    for (int q = 0; q < B; q++) xc[u][q] = j[u] != i ? ld_coherent(out + (size_t)j[u] * B + q) : 0.0;
-                    if constexpr (constexpr_is_half<V>::value) {
-                        // FP16: elements 2w and 2w + 1 of a block in one
-                        // 32-bit word (a zero high half past the last), so
-                        // the loads are whole words
-                        constexpr int NW = (B * B + 1) / 2;
-                        const __half2 *vw = reinterpret_cast<const __half2 *>(val) + (size_t)(k + u) * NW * WAVE + lane;
-#pragma unroll
-                        for (int w = 0; w < NW; w++) {
-                            const __half2 h = j[u] != i ? vw[w * WAVE] : __half2{};
-                            m[u][2 * w] = (double)__low2float(h);
-                            if (2 * w + 1 < B * B) m[u][2 * w + 1] = (double)__high2float(h);
-                        }
-                    } else {
-                        const V *vv = val + (size_t)(k + u) * B * B * WAVE + lane;
-#pragma unroll
-                        for (int q = 0; q < B * B; q++) m[u][q] = j[u] != i ? (double)cvt(vv[q * WAVE]) : 0.0;
+                    for (int w = 0; w < NW; w++) {
+                        const __half2 h = vw[w * WAVE];
+                        m[u][2 * w] = (double)__low2float(h);
+                        if (2 * w + 1 < B * B) m[u][2 * w + 1] = (double)__high2float(h);
                     }
-                }
+                } else {
+                    const V *vv = val + ks * B * B * WAVE + lane;
 #pragma unroll
-                for (int u = 0; u < BT_U; u++) {
-                    if (j[u] == i) continue;
-#pragma unroll
-                    for (int r = 0; r < B; r++) {
-#pragma unroll
-                        for (int q = 0; q < B; q++) acc[r] -= (sc * m[u][r * B + q]) * xc[u][q];
-                    }
+                    for (int q = 0; q < B * B; q++) m[u][q] = (double)cvt(vv[q * WAVE]);
                 }
             }
+            if (k == k0) wait_gate(sflag, gate, epoch);
+            read_results<BT_U, B, double>(out, j, use, xc, err);
+#pragma unroll
+            for (int u = 0; u < BT_U; u++) {
+                if (!use[u]) continue;
+#pragma unroll
+                for (int r = 0; r < B; r++) {
+#pragma unroll
+                    for (int q = 0; q < B; q++) acc[r] -= (sc * m[u][r * B + q]) * xc[u][q];
+                }
+            }
+        }
+        if (i >= 0) {
             if (dinv) {
 #pragma unroll
                 for (int r = 0; r < B; r++) {
                     double o = 0.0;
 #pragma unroll
                     for (int q = 0; q < B; q++) o += D[r * B + q] * acc[q];
-                    st_coherent(out + (size_t)i * B + r, o);
+                    st_result(out + (size_t)i * B + r, o);
                 }
             } else {
 #pragma unroll
-                for (int r = 0; r < B; r++) st_coherent(out + (size_t)i * B + r, acc[r]);
+                for (int r = 0; r < B; r++) st_result(out + (size_t)i * B + r, acc[r]);
             }
         }
-        st_flag_release(sflag + s, epoch);
+        raise_gate(sflag, s, epoch);
     }
 }
 
@@ -1352,39 +1492,6 @@ __global__ void __launch_bounds__(256) k_gs_chunk_grp(int n, int nchunks, int cp
     for (int r = threadIdx.x; r < row1 - row0; r += blockDim.x) un[row0 + r] = ux[r];
 }
 
-// Part of one row's Gauss-Seidel sum for a lane of a row group: entries
-// k, k + G, ... < ke of the plain CSR row i, only the dependent couplings
-// (DEP: j < i forward, j > i backward; x = the new values, read coherently)
-// or only the others (x = the entry values, ordinary loads).  U entries per
-// lane are loaded before any is used, then U gathers of x.
-template <int U, int G, typename V, typename X, bool DEP>
-__device__ __forceinline__ X gs_row_part(int k, int ke, int i, int dir, const int *__restrict__ ja,
-                                         const V *__restrict__ val, const X *x)
-{
-    X acc = 0;
-    for (; k < ke; k += U * G) {
-        int j[U];
-        V v[U];
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-            const int kk = k + u * G;
-            j[u] = kk < ke ? ja[kk] : -1;
-            v[u] = kk < ke ? val[kk] : (V)0;
-        }
-        X xv[U];
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-            const bool dep = dir > 0 ? j[u] < i : j[u] > i;
-            const bool use = j[u] >= 0 && j[u] != i && dep == DEP;
-            if (DEP) xv[u] = use ? ld_coherent(x + j[u]) : (X)0;
-            else xv[u] = use ? x[j[u]] : (X)0;
-        }
-#pragma unroll
-        for (int u = 0; u < U; u++) acc += (X)cvt(v[u]) * xv[u];
-    }
-    return acc;
-}
-
 // One Gauss-Seidel sweep as k_gs_sweep for levels with long rows: a slice
 // holds R = 64/G rows of one dependency level (perm[p] = row, -1 for
 // padding), each row summed by a group of G lanes over its plain CSR row
@@ -1409,17 +1516,35 @@ __global__ void __launch_bounds__(256) k_gs_sweep_grp(int nsl, const int *__rest
         if (s < 0 || s >= nsl) break;
         const int i = perm[s * R + lane / G];
         const int k0 = i >= 0 ? ia[i] + 1 + gl : 0, k1 = i >= 0 ? ia[i + 1] : 0;
-        X acc = uo ? gs_row_part<GRP_U, G, V, X, false>(k0, k1, i, dir, ja, val, uo) : (X)0;
-        wait_slices(dep_ptr, dep_list, sflag, s, epoch, lane, err);
-        acc += gs_row_part<GRP_U, G, V, X, true>(k0, k1, i, dir, ja, val, un);
-        acc = group_sum<G>(acc);
-        if (i >= 0 && gl == 0) {
-            const X d = diag[i];
-            const X sc = row_scaled<V>::value ? (X)rsc[i] : (X)1;
-            const X res = f[(size_t)i * fs] - sc * acc;
-            st_coherent(un + i, d != (X)0 ? res / d : (uo ? uo[i] : (X)0));
+        X d = 1, sc = 1, fi = 0, uold_i = 0;
+        if (i >= 0) {
+            d = diag[i];
+            fi = f[(size_t)i * fs];
+            if (uo) uold_i = uo[i];
+            if (row_scaled<V>::value) sc = (X)rsc[i];
         }
-        st_flag_release(sflag + s, epoch);
+        typedef gs_batch<GRP_U, G, 1, V, X> batch;
+        batch first;
+        first.load(k0, k1, 0, ja, val);
+        X acc = 0;
+        if (uo) {
+            acc = first.others(i, dir, uo);
+            for (int k = k0 + GRP_U * G; k < k1; k += GRP_U * G) {
+                batch t;
+                t.load(k, k1, 0, ja, val);
+                acc += t.others(i, dir, uo);
+            }
+        }
+        wait_gate(sflag, gate_slice(dep_ptr, dep_list, s, lane), epoch);
+        acc += first.dependencies(i, dir, un, err);
+        for (int k = k0 + GRP_U * G; k < k1; k += GRP_U * G) {
+            batch t;
+            t.load(k, k1, 0, ja, val);
+            acc += t.dependencies(i, dir, un, err);
+        }
+        acc = group_sum<G>(acc);
+        if (i >= 0 && gl == 0) st_result(un + i, d != (X)0 ? (fi - sc * acc) / d : uold_i);
+        raise_gate(sflag, s, epoch);
     }
 }
 
@@ -1985,6 +2110,14 @@ int jxamd_sweep_waves(int nsl)
     return nsl < cap ? (nsl > 0 ? nsl : 1) : cap;
 }
 
+// arms what a sync-free launch fills: b values of each row in perm (nullptr: y[0..npos-1])
+static void arm(int xt, long long npos, int b, const int *perm, void *y, hipStream_t st)
+{
+    const unsigned grid = (unsigned)((npos + 255) / 256);
+    if (xt == JXAMD_T_F64) k_arm<double><<<grid, 256, 0, st>>>(npos, b, perm, (double *)y);
+    else k_arm<float><<<grid, 256, 0, st>>>(npos, b, perm, (float *)y);
+}
+
 int jxamd_k_gs_sweep(int vt, int xt, int nsl, const int *perm, const int *sptr, const int *col, const void *val,
                      const float *rsc, const void *diag, const void *f, int fs, const void *uo, void *un,
                      const int *dep_ptr, const int *dep_list, int *sflag, int epoch, int dir,
@@ -1993,6 +2126,7 @@ int jxamd_k_gs_sweep(int vt, int xt, int nsl, const int *perm, const int *sptr, 
     if (nsl == 0) return 0;
     const int waves = jxamd_sweep_waves(nsl);
     const int grid = (waves + 3) / 4;
+    arm(xt, (long long)nsl * WAVE, 1, perm, un, (hipStream_t)stream);
     DISPATCH_VX(vt, xt,
                 (k_gs_sweep<V_, X_><<<grid, 256, 0, (hipStream_t)stream>>>(
                     nsl, perm, sptr, col, (const V_ *)val, rsc, (const X_ *)diag, (const X_ *)f, fs, (const X_ *)uo,
@@ -2077,16 +2211,14 @@ int jxamd_k_bhgs_multi(int b, int nsl, int K, const int *vorder, const int *perm
     const int grid = (waves + 3) / 4;
     hipStream_t st = (hipStream_t)stream;
     const unsigned long long b0 = *base;
-#define LAUNCH_BHGS(BS)                                                                                                \
-    k_bhgs_multi<BS><<<grid, 256, 0, st>>>(nsl, nvs, vorder, perm, sptr, col, val, dinv, rhs, xsl0, xs, xstride,      \
-                                           xout, dlo_ptr, dlo_list, dall_ptr, dall_list, sflag, epoch, w, omega,       \
-                                           ticket, b0, err)
-    switch (b) {
-    case 2: LAUNCH_BHGS(2); break;
-    case 3: LAUNCH_BHGS(3); break;
-    case 4: LAUNCH_BHGS(4); break;
-    default: return JXAMD_ERROR_ARG;
-    }
+    if (b < 2 || b > 4) return JXAMD_ERROR_ARG;
+    arm(JXAMD_T_F64, xstride * K, 1, nullptr, xs, st);
+#define LAUNCH_BHGS(BS, US)                                                                                            \
+    k_bhgs_multi<BS, US><<<grid, 256, 0, st>>>(nsl, nvs, vorder, perm, sptr, col, val, dinv, rhs, xsl0, xs, xstride,  \
+                                               xout, dlo_ptr, dlo_list, sflag, epoch, w, omega, ticket, b0, err)
+    if (b == 2) LAUNCH_BHGS(2, 6);
+    else if (b == 3) LAUNCH_BHGS(3, 6);
+    else LAUNCH_BHGS(4, 3);
 #undef LAUNCH_BHGS
     *base += (unsigned long long)nvs + (unsigned long long)grid * 4;
     return chk(hipGetLastError());
@@ -2164,6 +2296,7 @@ int jxamd_k_btri(int b, int vt, int nsl, const int *perm, const int *sptr, const
     const int waves = jxamd_sweep_waves(nsl);
     const int grid = (waves + 3) / 4;
     hipStream_t st = (hipStream_t)stream;
+    arm(JXAMD_T_F64, (long long)nsl * WAVE, b, perm, out, st);
     const unsigned long long b0 = *base;
 #define LAUNCH_BTRI(VT, DT)                                                                                            \
     do {                                                                                                               \
@@ -2306,6 +2439,7 @@ int jxamd_k_gs_sweep_grp(int G, int vt, int xt, int nsl, const int *perm, const 
     const int waves = jxamd_sweep_waves(nsl);
     const int grid = (waves + 3) / 4;
     hipStream_t st = (hipStream_t)stream;
+    arm(xt, (long long)nsl * (WAVE / G), 1, perm, un, st);
     DISPATCH_G(G, DISPATCH_VX(vt, xt,
                               (k_gs_sweep_grp<G_, V_, X_><<<grid, 256, 0, st>>>(
                                   nsl, perm, ia, ja, (const V_ *)val, rsc, (const X_ *)diag, (const X_ *)f, fs,

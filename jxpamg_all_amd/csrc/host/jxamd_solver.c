@@ -1836,7 +1836,7 @@ static int lds_build(const jxamd_solver *s, const jxamd_csr *A, const int *ord, 
  * workgroup is the faster.  Measured: a step of W wavefronts with U entries
  * per lane takes 0.2 + 0.0075 U W us (barrier, gathers, division; the
  * wavefronts' instructions), records beyond the L2 come at some 45 GB/s;
- * k_gs_sweep takes about 3 us per dependency level on the whole device. */
+ * k_gs_sweep takes about 2.3 us per dependency level on the whole device. */
 static int build_lds(jxamd_solver *s, int l, const jxamd_csr *A)
 {
     dlds *g = &s->Gl[l];
@@ -1848,7 +1848,7 @@ static int build_lds(jxamd_solver *s, int l, const jxamd_csr *A)
         e = ord[d] ? lds_levels(A, d ? -1 : 1, ord[d], &start[d], &nl[d]) : JXAMD_ERROR_MEMORY;
     }
     if (!e && nl[0] && nl[1]) {
-        double best = 3.0 * nl[0];
+        double best = 2.3 * nl[0];
         int G = 0, U = 0, W = 0;
         for (int g1 = 1; g1 <= 16; g1 *= 2)
             for (int u1 = 4; u1 <= 8; u1 += 4)
