@@ -71,34 +71,43 @@ int jxamd_k_gs_sweep_grp(int G, int vt, int xt, int nsl, const int *perm, const 
                          void *un, const int *dep_ptr, const int *dep_list, int *sflag, int epoch, int dir,
                          unsigned long long *ticket, unsigned long long *base, int *err, void *stream);
 /* Exact relax-6 sweeps of a small level in one workgroup, the vector in LDS
- * (k_gs_lds).  A direction's schedule is a list of steps; in step t wavefront
- * w of `waves` works on a record: 64/G rows of one dependency level, G lanes
- * per row, U entries per lane (padding: value 0, column n).  Rows of more than
- * G * U entries take several records in consecutive steps.  Place t * waves + w
- * of the schedule names the rows and the record (record 0, all padding, where
- * a wavefront has nothing to do).  JXAMD_LDS_AHEAD steps of padding follow the
- * last.  Entries lie in 16-byte
- * vectors: entry u of a lane is component u % E of vector u / E, E = 16 /
- * sizeof(value) for the values, 4 for the columns, which are byte offsets
- * into the vector. */
-#define JXAMD_LDS_NONE 0xffffff  /* row number of padding */
-#define JXAMD_LDS_LAST 0x1000000 /* the rows' last record: the new values are formed */
-#define JXAMD_LDS_CONT 0x2000000 /* the rows' sums go on from the previous record */
-#define JXAMD_LDS_AHEAD 4
+ * (k_gs_lds).  The rows are taken in the order of their dependency levels
+ * (order[q]: row at place q); a slice is 64/G consecutive places of one
+ * level.  A direction's schedule is a list of steps; in step t wavefront w of
+ * `waves` works on a record: a slice with G lanes per row and U entries per
+ * lane (padding: value 0, column n), of the couplings the direction depends on
+ * (columns below the row forward, above it backward).  Slices with rows of
+ * more than G * U such entries take several records in consecutive steps.
+ * Entry t * waves + w of the schedule is a pair: the slice's first place,
+ * its number of rows and flags, and the record (0 rows and record 0, all
+ * padding, where a wavefront has nothing to do).  2 JXAMD_LDS_DEPTH steps of
+ * padding follow the last.  Entries lie in 16-byte vectors: entry u of a lane
+ * is component u % E of vector u / E, E = 16 / sizeof(value) for the values,
+ * 4 for the columns, which are places as byte offsets into the vector. */
+#define JXAMD_LDS_ROW 0xffff
+#define JXAMD_LDS_COUNT(e) (((e) >> 16) & 0x7f)
+#define JXAMD_LDS_LAST 0x1000000 /* the slice's last record: the new values are formed */
+#define JXAMD_LDS_CONT 0x2000000 /* the sums go on from the previous record */
+#define JXAMD_LDS_DEPTH 4 /* records a wavefront holds; steps come in multiples of it */
+#define JXAMD_LDS_PAD 64  /* values behind the last row's in diag and work that may be read */
+/* most wavefronts: with U = 8, four FP64 records fill more than the 128 registers that 16 leave a lane */
+#define JXAMD_LDS_WAVES(U, xt) ((U) == 8 && (xt) == JXAMD_T_F64 ? 8 : 16)
 typedef struct {
-    const int *row;            /* pairs (place * 64/G + r): row with the flags (the same in every r), record */
+    const int *sched;
     const unsigned int *col;   /* vector h of lane: (rec * U/4 + h) * 64 + lane */
     const void *val;           /* vector h of lane: (rec * U/E + h) * 64 + lane */
-    const void *diag;          /* a_ii and 1 / a_ii: diag[2 (rec * 64/G + r)] (a_ii = 0: the row keeps its value) */
-    int steps;                 /* a multiple of three */
+    int steps;
 } jxamd_lds_sweep;
 /* rows of vector type xt that fit the device's LDS (0: not available); a
  * device layer without these two leaves them undefined, and the solver then
  * keeps to jxamd_k_gs_sweep */
 int jxamd_gs_lds_rows(int xt) __attribute__((weak));
-/* ncalls relax-6 calls (forward, then backward sweep) from uo (NULL: zeros) into un */
+/* ncalls relax-6 calls (forward, then backward sweep) from uo (NULL: zeros)
+ * into un; diag: a_ii and 1 / a_ii of place q at 2 q (a_ii = 0: the row keeps
+ * its value); work: 2 (n + JXAMD_LDS_PAD) values of type xt */
 int jxamd_k_gs_lds(int G, int U, int waves, int xt, int n, const jxamd_lds_sweep *fw, const jxamd_lds_sweep *bw,
-                   int ncalls, const void *f, int fs, const void *uo, void *un, void *stream) __attribute__((weak));
+                   const int *order, const void *diag, int ncalls, const void *f, int fs, const void *uo, void *un,
+                   void *work, void *stream) __attribute__((weak));
 /* stage 2: x^(-1) into slice order, then K fused sweeps (columns of the
  * layout are positions, ~pos for lower neighbours; xs holds K slice-ordered
  * vectors of xstride doubles; the last sweep also writes xout in row order) */

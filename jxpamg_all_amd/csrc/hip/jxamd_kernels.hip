@@ -18,6 +18,7 @@
 #include <hip/hip_fp16.h>
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <type_traits>
 
 #define WAVE 64
 #define SPIN_LIMIT (1 << 24)
@@ -657,95 +658,124 @@ template <int G, typename X> __device__ __forceinline__ X dpp_sum(X v)
 }
 
 // Exact relax-6 sweeps of a level whose vector fits in LDS: one workgroup,
-// the vector updated in place (the host has checked that a row's couplings
-// all lie on other dependency levels: the earlier ones hold new values, the
-// later ones still their old ones).  A dependency level is one step, or a few, and
-// costs a workgroup barrier, LDS gathers, a division and an LDS store, where
-// k_gs_sweep pays a round trip through the device's coherence point (2 us).  The steps' records do not depend on x: a wavefront holds
-// three in registers, refilled as they are used, so that the loads of a step
-// are issued three steps ahead.
+// the vector updated in place, rows in the order of their dependency levels
+// (the host has checked that a row's couplings all lie on other levels and
+// that the levels, backwards, are those of the backward sweep).  A dependency
+// level is one step, or a few, and costs a workgroup barrier, LDS gathers, a
+// division and an LDS store, where k_gs_sweep pays a round trip through the
+// device's coherence point (2 us).  The steps' records do not depend on x: a
+// wavefront holds four in registers, refilled as they are used, so that the
+// loads of a step are issued three steps ahead, and its place in the schedule seven.
 // Only LDS is ordered at a step's end: the loads stay in flight across it.
-// All sweeps of a level visit run in one launch.  Per sweep, with a flag-per-slice
-// k_gs_sweep before: 20160 rows of 7 (83 levels) 60 us, 253 before; 8807 rows of 23 (261
-// levels) 153 and 835; 2114 rows of 61 (374 levels) 115 and 1130; 2048 rows
-// of 7 (38 levels) 12 and 102.
-// A step's time is its wavefronts' instructions as much as its latencies
-// (0.35 us with 8-byte loads, packed columns and the compiler's division at
-// G 16, U 8, two wavefronts), hence 16-byte loads at scalar base + lane offset,
-// columns as LDS byte offsets, and the quotient from the stored reciprocal.
-#define LDS_P 3
+// All sweeps of a level visit run in one launch, and a sweep reads only the
+// entries of its dependencies: the sum over a row's other couplings is the one
+// the sweep before it formed when it passed the row, since none of them has
+// changed after that.  h keeps f less that sum; the first sweep finds it in
+// a pass without barriers, or starts from f where the entry vector is zero.
+// f and h lie in the rows' order, too: loads by row number take a cycle per
+// lane (336 us instead of 196 for the first level below).
+// Two calls (four sweeps), with a flag-per-slice k_gs_sweep, with full rows
+// in LDS and now: 20160 rows of 7 (83 levels) 1010, 240 and 196 us; 8807 rows
+// of 23 (261 levels) 3340, 609 and 499; 2114 rows of 61 (374 levels) 4520, 456
+// and 430; 2048 rows of 7 (38 levels) 408, 46 and 39.
+// A step's time is its wavefronts' instructions as much as its latencies,
+// hence 16-byte loads at scalar base + lane offset, columns as LDS byte
+// offsets, and the quotient from the stored reciprocal.
+#define LDS_P JXAMD_LDS_DEPTH
 
-// a / d with rd = 1 / d rounded: one correction by the exact remainder makes
-// the product the rounded quotient (but for underflow); a remainder that is not finite (a or
-// the quotient infinite or NaN, or 1 / d overflowed) takes the division
-template <typename X> __device__ __forceinline__ X div_by(X a, X d, X rd)
+template <int G, int U, int MAXW, typename X>
+__global__ void __launch_bounds__(WAVE *MAXW) k_gs_lds(int n, jxamd_lds_sweep fw, jxamd_lds_sweep bw,
+                                                       const int *__restrict__ order, const X *diag, int npass,
+                                                       const X *__restrict__ f, int fs, const X *uo, X *un, X *work)
 {
-    const X q = a * rd;
-    const X r = fma(-d, q, a);
-    if (__builtin_expect(!(fabs(r) < (X)__builtin_huge_val()), 0)) return a / d;
-    return fma(r, rd, q);
-}
-
-template <int G, int U, typename X>
-__global__ void __launch_bounds__(1024) k_gs_lds(int n, jxamd_lds_sweep fw, jxamd_lds_sweep bw, int npass, const X *f,
-                                                 int fs, const X *uo, X *un)
-{
-    constexpr int R = WAVE / G;
     typedef typename vec16<X>::T XV;
     typedef unsigned int __attribute__((ext_vector_type(4))) UV;
     typedef X __attribute__((ext_vector_type(2))) X2;
     constexpr int E = 16 / sizeof(X), NV = U / E, NC = U / 4;
     extern __shared__ __align__(16) unsigned char smraw[];
-    X *x = reinterpret_cast<X *>(smraw);
-    for (int i = threadIdx.x; i < n; i += blockDim.x) x[i] = uo ? uo[i] : (X)0;
+    X *x = reinterpret_cast<X *>(smraw), *fo = work, *h = work + n + JXAMD_LDS_PAD;
+    constexpr int BT = 8; // loads in flight per lane while f and u change order
+    const int step = blockDim.x;
+    for (int q0 = threadIdx.x; q0 < n; q0 += BT * step) {
+        int i[BT];
+        X a[BT], u[BT];
+#pragma unroll
+        for (int b = 0; b < BT; b++) i[b] = order[min(q0 + b * step, n - 1)];
+#pragma unroll
+        for (int b = 0; b < BT; b++) {
+            a[b] = f[(size_t)i[b] * fs];
+            u[b] = uo ? uo[i[b]] : (X)0;
+        }
+#pragma unroll
+        for (int b = 0; b < BT; b++)
+            if (q0 + b * step < n) {
+                fo[q0 + b * step] = a[b];
+                x[q0 + b * step] = u[b];
+            }
+    }
     if (threadIdx.x == 0) x[n] = 0; // the column of padding entries
     __syncthreads();
     const unsigned lane = threadIdx.x % WAVE, gl = lane % G, r = lane / G;
     const int W = blockDim.x / WAVE, w = wave_id();
-    for (int pass = 0; pass < npass; pass++) {
-        const jxamd_lds_sweep sw = pass & 1 ? bw : fw;
-        int row[LDS_P]; // of the records in registers
-        int2 ra;        // rows and record of the next refill
+    // one pass over a direction's steps.  SUM: only the rows' sums over the
+    // direction's dependencies at the present values, f - sum into h; else
+    // the sweep, from g = f less the sum over the other couplings
+    auto pass = [&](auto sum_only, const jxamd_lds_sweep &sw, const X *g, bool keep) {
+        constexpr bool SUM = decltype(sum_only)::value;
+        int2 ra[LDS_P]; // rows, flags and record of the refills to come
+        int fl[LDS_P];  // rows and flags of the records in registers
         X2 d[LDS_P];
-        X ff[LDS_P];
+        X ff[LDS_P], gg[LDS_P];
         XV v[LDS_P][NV];
         UV c[LDS_P][NC];
-        auto row_of = [&](int t) {
-            return *(const int2 *)((const char *)sw.row + ((size_t)t * W + w) * (R * sizeof(int2)) + r * sizeof(int2));
+        auto place = [&](int t) { return *(const int2 *)(sw.sched + 2 * ((size_t)t * W + w)); };
+        auto at = [&](const X *y, int e) { // y at the lane's row (JXAMD_LDS_PAD values follow the last)
+            return (const char *)y + (unsigned)(((e & JXAMD_LDS_ROW) + r) * sizeof(X));
         };
-        auto fill = [&](int p) {
-            const size_t rec = (size_t)__builtin_amdgcn_readfirstlane(ra.y);
-            row[p] = ra.x;
-            ff[p] = *(const X *)((const char *)f + __umul24(min(ra.x & JXAMD_LDS_NONE, n - 1), fs * (int)sizeof(X)));
-            d[p] = *(const X2 *)((const char *)sw.diag + rec * R * sizeof(X2) + r * sizeof(X2));
+        auto fill = [&](int p, bool with_g) {
+            const size_t rec = (size_t)__builtin_amdgcn_readfirstlane(ra[p].y);
+            fl[p] = __builtin_amdgcn_readfirstlane(ra[p].x);
+            ff[p] = *(const X *)at(fo, fl[p]);
+            if (!SUM && with_g) gg[p] = *(const X *)at(g, fl[p]);
+            if (!SUM) d[p] = *(const X2 *)((const char *)diag + (unsigned)(((fl[p] & JXAMD_LDS_ROW) + r) * sizeof(X2)));
             const char *cb = (const char *)sw.col + rec * (NC * WAVE * sizeof(UV));
             const char *vb = (const char *)sw.val + rec * (NV * WAVE * sizeof(XV));
 #pragma unroll
-            for (int h = 0; h < NC; h++) c[p][h] = *(const UV *)(cb + lane * sizeof(UV) + h * (WAVE * sizeof(UV)));
+            for (int q = 0; q < NC; q++) c[p][q] = *(const UV *)(cb + lane * sizeof(UV) + q * (WAVE * sizeof(UV)));
 #pragma unroll
-            for (int h = 0; h < NV; h++) v[p][h] = *(const XV *)(vb + lane * sizeof(XV) + h * (WAVE * sizeof(XV)));
+            for (int q = 0; q < NV; q++) v[p][q] = *(const XV *)(vb + lane * sizeof(XV) + q * (WAVE * sizeof(XV)));
         };
 #pragma unroll
-        for (int p = 0; p < LDS_P; p++) {
-            ra = row_of(p);
-            fill(p);
+        for (int p = 0; p < LDS_P; p++) ra[p] = place(p);
+#pragma unroll
+        for (int p = 0; p < LDS_P - 1; p++) {
+            fill(p, false);
+            ra[p] = place(LDS_P + p);
         }
-        ra = row_of(LDS_P);
+        __syncthreads(); // the pass before is over: its x and h are whole
+        if (!SUM) {
+#pragma unroll
+            for (int p = 0; p < LDS_P - 1; p++) gg[p] = *(const X *)at(g, fl[p]);
+        }
         __builtin_amdgcn_s_waitcnt(0); // the loop's waits then count only its own loads
         X acc = 0;
         for (int t = 0; t < sw.steps; t += LDS_P) {
 #pragma unroll
             for (int p = 0; p < LDS_P; p++) {
-                // loads return in order: the row number of the next refill
-                // goes before this step's record, so that waiting for it
-                // leaves the record's loads in flight
-                const int2 rn = row_of(t + p + LDS_P + 1);
-                const int fl = __builtin_amdgcn_readfirstlane(row[p]);
-                if (!(fl & JXAMD_LDS_CONT)) acc = 0;
+                const int e = fl[p];
+                if (!(e & JXAMD_LDS_CONT)) acc = 0;
                 X xv[U];
 #pragma unroll
                 for (int u = 0; u < U; u++) xv[u] = *reinterpret_cast<const X *>(smraw + c[p][u / 4][u % 4]);
                 __builtin_amdgcn_sched_barrier(0); // every gather issued before the first is waited for
+                // the record of step t + p + LDS_P - 1, into the registers of
+                // the step before, and the place of the one LDS_P on, issued
+                // while the gathers are on their way; loads return in order,
+                // so a step waits only for loads as old as its own record's
+                const int b = (p + LDS_P - 1) % LDS_P;
+                fill(b, true);
+                ra[b] = place(t + p + 2 * LDS_P - 1);
+                __builtin_amdgcn_sched_barrier(0);
                 X acc2 = 0;
 #pragma unroll
                 for (int u = 0; u < U; u += 2) {
@@ -753,20 +783,40 @@ __global__ void __launch_bounds__(1024) k_gs_lds(int n, jxamd_lds_sweep fw, jxam
                     acc2 += v[p][(u + 1) / E][(u + 1) % E] * xv[u + 1];
                 }
                 acc += acc2;
-                if (fl & JXAMD_LDS_LAST) {
+                if (e & JXAMD_LDS_LAST) {
                     const X sum = dpp_sum<G>(acc);
-                    // a row with a zero diagonal keeps its value
-                    const int i = row[p] & JXAMD_LDS_NONE;
-                    if (gl == 0 && i < n && d[p][0] != (X)0) x[i] = div_by(ff[p] - sum, d[p][0], d[p][1]);
+                    const bool in = gl == 0 && r < (unsigned)JXAMD_LDS_COUNT(e);
+                    const unsigned i = (e & JXAMD_LDS_ROW) + r;
+                    if (!SUM) {
+                        // a / d from rd = 1 / d rounded: one correction by
+                        // the exact remainder makes the product the rounded
+                        // quotient (but for underflow); where a remainder is
+                        // not finite (a or the quotient infinite or NaN, or
+                        // 1 / d overflowed) the wavefront divides.  A row
+                        // with a zero diagonal keeps its value.
+                        const X a = gg[p] - sum, di = d[p][0], rd = d[p][1], q = a * rd, rem = fma(-di, q, a);
+                        const bool wr = in && di != (X)0;
+                        X xn = fma(rem, rd, q);
+                        if (__builtin_expect(__ballot(wr && !(fabs(rem) < (X)__builtin_huge_val())) != 0, 0)) xn = a / di;
+                        if (wr) x[i] = xn;
+                    }
+                    if ((SUM || keep) && in) h[i] = ff[p] - sum;
                 }
-                fill(p);
-                ra = rn;
-                asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+                if (!SUM) asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
             }
         }
-    }
+    };
+    if (uo) pass(std::true_type{}, bw, nullptr, true);
+    for (int q = 0; q < npass; q++) pass(std::false_type{}, q & 1 ? bw : fw, q > 0 || uo ? h : fo, q + 1 < npass);
     __syncthreads();
-    for (int i = threadIdx.x; i < n; i += blockDim.x) un[i] = x[i];
+    for (int q0 = threadIdx.x; q0 < n; q0 += BT * step) {
+        int i[BT];
+#pragma unroll
+        for (int b = 0; b < BT; b++) i[b] = order[min(q0 + b * step, n - 1)];
+#pragma unroll
+        for (int b = 0; b < BT; b++)
+            if (q0 + b * step < n) un[i[b]] = x[q0 + b * step];
+    }
 }
 
 // K forward block hybrid SOR sweeps on the BSR matrix in one launch
@@ -2143,30 +2193,32 @@ int jxamd_gs_lds_rows(int xt)
         return 0;
     const size_t xsz = xt == JXAMD_T_F64 ? sizeof(double) : sizeof(float);
     const long rows = (long)(lds / xsz) - 1; // and the padding column
-    return (int)(rows > 65535 ? 65535 : (rows < 0 ? 0 : rows)); // row * fs * size is a 24-bit product
+    return (int)(rows > JXAMD_LDS_ROW ? JXAMD_LDS_ROW : (rows < 0 ? 0 : rows));
 }
 
 int jxamd_k_gs_lds(int G, int U, int waves, int xt, int n, const jxamd_lds_sweep *fw, const jxamd_lds_sweep *bw,
-                   int ncalls, const void *f, int fs, const void *uo, void *un, void *stream)
+                   const int *order, const void *diag, int ncalls, const void *f, int fs, const void *uo, void *un,
+                   void *work, void *stream)
 {
     if (n < 1 || ncalls < 1) return 0;
-    if (waves < 1 || waves > 16 || n > jxamd_gs_lds_rows(xt) || fs < 1 || fs > 1024) return JXAMD_ERROR_ARG;
+    if (waves < 1 || waves > JXAMD_LDS_WAVES(U, xt) || n > jxamd_gs_lds_rows(xt)) return JXAMD_ERROR_ARG;
     if (fw->steps % LDS_P || bw->steps % LDS_P) return JXAMD_ERROR_ARG;
     const size_t lds = ((size_t)n + 1) * (xt == JXAMD_T_F64 ? sizeof(double) : sizeof(float));
     hipStream_t st = (hipStream_t)stream;
-#define LAUNCH_GL(GG, UU, XX)                                                                                          \
+#define LAUNCH_GL(GG, UU, XX, TT)                                                                                      \
     do {                                                                                                               \
-        const hipError_t e_ = hipFuncSetAttribute((const void *)k_gs_lds<GG, UU, XX>,                                  \
-                                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);               \
-        if (e_ != hipSuccess) return JXAMD_ERROR_DEVICE;                                                               \
-        k_gs_lds<GG, UU, XX><<<1, waves * WAVE, lds, st>>>(n, *fw, *bw, 2 * ncalls, (const XX *)f, fs, (const XX *)uo, \
-                                                           (XX *)un);                                                  \
+        auto kern_ = k_gs_lds<GG, UU, JXAMD_LDS_WAVES(UU, TT), XX>;                                                    \
+        if (hipFuncSetAttribute((const void *)kern_, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) !=         \
+            hipSuccess)                                                                                                \
+            return JXAMD_ERROR_DEVICE;                                                                                 \
+        kern_<<<1, waves * WAVE, lds, st>>>(n, *fw, *bw, order, (const XX *)diag, 2 * ncalls, (const XX *)f, fs,       \
+                                            (const XX *)uo, (XX *)un, (XX *)work);                                     \
         return chk(hipGetLastError());                                                                                 \
     } while (0)
 #define LAUNCH_GX(GG, UU)                                                                                              \
     do {                                                                                                               \
-        if (xt == JXAMD_T_F64) LAUNCH_GL(GG, UU, double);                                                             \
-        else LAUNCH_GL(GG, UU, float);                                                                                 \
+        if (xt == JXAMD_T_F64) LAUNCH_GL(GG, UU, double, JXAMD_T_F64);                                                \
+        else LAUNCH_GL(GG, UU, float, JXAMD_T_F32);                                                                    \
     } while (0)
 #define LAUNCH_GU(GG)                                                                                                  \
     do {                                                                                                               \

@@ -80,6 +80,8 @@ typedef struct {
 typedef struct {
     int G, U, W;
     jxamd_lds_sweep sw[2]; /* forward, backward */
+    int *order;
+    void *diag, *work;
     double abytes;         /* algorithmic bytes of one sweep */
 } dlds;
 
@@ -1696,32 +1698,58 @@ static int build_poly(jxamd_solver *s, int l, const jxamd_hierarchy *H)
     return e;
 }
 
-/* Rows by dependency level of one direction (ord, level l at start[l] ..
- * start[l + 1], longer rows first inside a level) for sweeps that update one
- * vector in place: beside the dependencies, which lie on earlier levels, every
- * other coupling of a row must lie on a later one (it does for a symmetric
- * pattern), or the row would read a value that is already new.  *nlev = 0
- * where that does not hold. */
-static int lds_levels(const jxamd_csr *A, int dir, int *ord, int **ostart, int *nlev)
+/* The couplings of one direction's dependencies (j < i forward, j > i
+ * backward), rows as CSR without the diagonal. */
+static int lds_deps(const jxamd_csr *A, int dir, jxamd_csr *D)
 {
     const int n = A->n;
+    memset(D, 0, sizeof(*D));
+    int *ia = (int *)malloc(sizeof(int) * ((size_t)n + 1));
+    int *ja = (int *)malloc(sizeof(int) * (size_t)(A->ia[n] + 1));
+    double *a = (double *)malloc(sizeof(double) * (size_t)(A->ia[n] + 1));
+    if (!ia || !ja || !a) { free(ia); free(ja); free(a); return JXAMD_ERROR_MEMORY; }
+    int q = 0;
+    for (int i = 0; i < n; i++) {
+        ia[i] = q;
+        for (int k = A->ia[i] + 1; k < A->ia[i + 1]; k++)
+            if (dir > 0 ? A->ja[k] < i : A->ja[k] > i) {
+                ja[q] = A->ja[k];
+                a[q++] = A->a[k];
+            }
+    }
+    ia[n] = q;
+    D->n = D->ncols = n;
+    D->ia = ia;
+    D->ja = ja;
+    D->a = a;
+    return 0;
+}
+
+/* Rows by dependency level of the forward sweep (F, B: the forward and the
+ * backward dependencies; ord, level l at start[l] .. start[l + 1], longer rows
+ * first inside a level) for sweeps that update one vector in place: the
+ * backward dependencies of a row must lie on later levels (they do for a
+ * symmetric pattern), or the forward sweep would read values that are already
+ * new, and the levels, backwards, would not order the backward sweep.
+ * *nlev = 0 where that does not hold. */
+static int lds_levels(const jxamd_csr *F, const jxamd_csr *B, int *ord, int **ostart, int *nlev)
+{
+    const int n = F->n;
     int *lev = (int *)malloc(sizeof(int) * (size_t)n);
     if (!lev) return JXAMD_ERROR_MEMORY;
     int nl = 0, maxlen = 0, ok = 1;
-    for (int t = 0; t < n; t++) {
-        const int i = dir > 0 ? t : n - 1 - t;
+#define LDS_ROW_LEN(i) (F->ia[(i) + 1] - F->ia[i] + B->ia[(i) + 1] - B->ia[i])
+    for (int i = 0; i < n; i++) {
         int l = 0;
-        for (int k = A->ia[i]; k < A->ia[i + 1]; k++) {
-            const int j = A->ja[k];
-            if ((dir > 0 ? j < i : j > i) && lev[j] + 1 > l) l = lev[j] + 1;
-        }
+        for (int k = F->ia[i]; k < F->ia[i + 1]; k++)
+            if (lev[F->ja[k]] + 1 > l) l = lev[F->ja[k]] + 1;
         lev[i] = l;
         if (l + 1 > nl) nl = l + 1;
-        if (A->ia[i + 1] - A->ia[i] > maxlen) maxlen = A->ia[i + 1] - A->ia[i];
+        if (LDS_ROW_LEN(i) > maxlen) maxlen = LDS_ROW_LEN(i);
     }
     for (int i = 0; i < n && ok; i++)
-        for (int k = A->ia[i]; k < A->ia[i + 1]; k++)
-            if ((dir > 0 ? A->ja[k] > i : A->ja[k] < i) && lev[A->ja[k]] <= lev[i]) ok = 0;
+        for (int k = B->ia[i]; k < B->ia[i + 1]; k++)
+            if (lev[B->ja[k]] <= lev[i]) ok = 0;
     *nlev = 0;
     *ostart = NULL;
     if (!ok) { free(lev); return 0; }
@@ -1729,9 +1757,10 @@ static int lds_levels(const jxamd_csr *A, int dir, int *ord, int **ostart, int *
     int *bylen = (int *)malloc(sizeof(int) * (size_t)n);
     int *cnt = (int *)calloc((size_t)(maxlen > nl ? maxlen : nl) + 2, sizeof(int));
     if (!start || !bylen || !cnt) { free(lev); free(start); free(bylen); free(cnt); return JXAMD_ERROR_MEMORY; }
-    for (int i = 0; i < n; i++) cnt[maxlen - (A->ia[i + 1] - A->ia[i]) + 1]++;
+    for (int i = 0; i < n; i++) cnt[maxlen - LDS_ROW_LEN(i) + 1]++;
     for (int q = 0; q <= maxlen; q++) cnt[q + 1] += cnt[q];
-    for (int i = 0; i < n; i++) bylen[cnt[maxlen - (A->ia[i + 1] - A->ia[i])]++] = i;
+    for (int i = 0; i < n; i++) bylen[cnt[maxlen - LDS_ROW_LEN(i)]++] = i;
+#undef LDS_ROW_LEN
     for (int i = 0; i < n; i++) start[lev[i] + 1]++;
     for (int l = 0; l < nl; l++) start[l + 1] += start[l];
     for (int l = 0; l < nl; l++) cnt[l] = start[l];
@@ -1744,128 +1773,144 @@ static int lds_levels(const jxamd_csr *A, int dir, int *ord, int **ostart, int *
     return 0;
 }
 
-/* steps of a schedule: a level's rows in slices of R, W slices at a time, a
- * slice taking one record (in consecutive steps) per G * U entries of its
- * longest row */
-static long lds_steps(const jxamd_csr *A, const int *ord, const int *start, int nl, int G, int U, int W, long *nrec)
+/* records of the slice at places b .. e: one per G * U entries of its longest row */
+static int lds_records(const jxamd_csr *D, const int *ord, int b, int e, int GU)
+{
+    int len = 1;
+    for (; b < e; b++)
+        if (D->ia[ord[b] + 1] - D->ia[ord[b]] > len) len = D->ia[ord[b] + 1] - D->ia[ord[b]];
+    return (len + GU - 1) / GU;
+}
+
+/* steps of a direction's schedule: a level's slices of R rows, W at a time, as
+ * many steps as the slice with most records has */
+static long lds_steps(const jxamd_csr *D, const int *ord, const int *start, int nl, int G, int U, int W, long *nrec)
 {
     const int R = SELLW / G;
     long steps = 0, recs = 1;
     for (int l = 0; l < nl; l++)
-        for (int b = start[l]; b < start[l + 1]; b += R) { /* longest row first */
-            const int len = A->ia[ord[b] + 1] - A->ia[ord[b]] - 1, ns = len > G * U ? (len + G * U - 1) / (G * U) : 1;
-            recs += ns;
-            if ((b - start[l]) / R % W == 0) steps += ns;
+        for (int b = start[l]; b < start[l + 1];) {
+            int most = 0;
+            for (int w = 0; w < W && b < start[l + 1]; w++, b += R) {
+                const int ns = lds_records(D, ord, b, b + R < start[l + 1] ? b + R : start[l + 1], G * U);
+                recs += ns;
+                if (ns > most) most = ns;
+            }
+            steps += most;
         }
     *nrec = recs;
     return steps;
 }
 
-/* the schedule and records of one direction, uploaded */
-static int lds_build(const jxamd_solver *s, const jxamd_csr *A, const int *ord, const int *start, int nl, int G, int U,
-                     int W, jxamd_lds_sweep *o)
+/* the schedule and records of one direction (dependencies D), uploaded */
+static int lds_build(const jxamd_solver *s, const jxamd_csr *D, int dir, const int *ord, const int *place,
+                     const int *start, int nl, int G, int U, int W, jxamd_lds_sweep *o)
 {
-    const int R = SELLW / G, n = A->n, xsz = (int)s->xsz, E = 16 / xsz;
-    long nrec = 0, steps = lds_steps(A, ord, start, nl, G, U, W, &nrec);
-    steps = (steps + 2) / 3 * 3;
-    const size_t recs = (size_t)nrec, places = (size_t)(steps + JXAMD_LDS_AHEAD) * W;
-    int *row = (int *)malloc(sizeof(int) * 2 * places * R);
-    double *diag = (double *)malloc(sizeof(double) * 2 * recs * R);
+    const int R = SELLW / G, n = D->n, xsz = (int)s->xsz, E = 16 / xsz;
+    long nrec = 0, steps = lds_steps(D, ord, start, nl, G, U, W, &nrec);
+    steps = (steps + JXAMD_LDS_DEPTH - 1) / JXAMD_LDS_DEPTH * JXAMD_LDS_DEPTH;
+    const size_t recs = (size_t)nrec, places = (size_t)(steps + 2 * JXAMD_LDS_DEPTH) * W;
+    int *sched = (int *)calloc(2 * places, sizeof(int));
     int *col = (int *)malloc(sizeof(int) * recs * U * SELLW);
     double *val = (double *)calloc(recs * U * SELLW, sizeof(double));
-    int e = !row || !diag || !col || !val ? JXAMD_ERROR_MEMORY : 0;
+    int e = !sched || !col || !val ? JXAMD_ERROR_MEMORY : 0;
     if (!e) {
-        for (size_t q = 0; q < places * R; q++) {
-            row[2 * q] = JXAMD_LDS_NONE;
-            row[2 * q + 1] = 0;
-        }
-        for (size_t q = 0; q < 2 * recs * R; q++) diag[q] = 1.0;
         for (size_t q = 0; q < recs * U * SELLW; q++) col[q] = n * xsz;
         size_t t = 0, rec = 1;
-        for (int l = 0; l < nl; l++)
-            for (int b = start[l]; b < start[l + 1]; b += R * W) {
-                int tmax = 1;
-                for (int w = 0; w < W; w++) {
-                    const int b0 = b + w * R;
-                    if (b0 >= start[l + 1]) break;
-                    const int len0 = A->ia[ord[b0] + 1] - A->ia[ord[b0]] - 1;
-                    const int ns = len0 > G * U ? (len0 + G * U - 1) / (G * U) : 1;
-                    if (ns > tmax) tmax = ns;
+        for (int ll = 0; ll < nl; ll++) {
+            const int l = dir > 0 ? ll : nl - 1 - ll, end = start[l + 1];
+            for (int b = start[l]; b < end;) {
+                int most = 0;
+                for (int w = 0; w < W && b < end; w++, b += R) {
+                    const int cnt = b + R < end ? R : end - b, ns = lds_records(D, ord, b, b + cnt, G * U);
+                    if (ns > most) most = ns;
                     for (int h = 0; h < ns; h++, rec++) {
-                        const size_t place = (t + h) * W + w;
-                        const int fl = (h > 0 ? JXAMD_LDS_CONT : 0) | (h == ns - 1 ? JXAMD_LDS_LAST : 0);
-                        for (int r = 0; r < R; r++) {
-                            row[2 * (place * R + r)] |= fl;
-                            row[2 * (place * R + r) + 1] = (int)rec;
-                            if (b0 + r >= start[l + 1]) continue;
-                            const int i = ord[b0 + r], k0 = A->ia[i] + 1, len = A->ia[i + 1] - k0;
-                            row[2 * (place * R + r)] = i | fl;
-                            /* the diagonal as the kernel holds it, and its reciprocal */
-                            const double di = s->xt == JXAMD_T_F64 ? A->a[A->ia[i]] : (double)(float)A->a[A->ia[i]];
-                            diag[2 * (rec * R + r)] = di;
-                            diag[2 * (rec * R + r) + 1] = di != 0.0 ? 1.0 / di : 0.0;
+                        int *q = sched + 2 * ((t + h) * W + w);
+                        q[0] = b | cnt << 16 | (h > 0 ? JXAMD_LDS_CONT : 0) | (h == ns - 1 ? JXAMD_LDS_LAST : 0);
+                        q[1] = (int)rec;
+                        for (int r = 0; r < cnt; r++) {
+                            const int i = ord[b + r], k0 = D->ia[i], len = D->ia[i + 1] - k0;
                             /* entry pp of the row: record pp / (G U), slot (pp / G) % U, lane pp % G */
                             for (int pp = h * G * U; pp < len && pp < (h + 1) * G * U; pp++) {
-                                if (A->ja[k0 + pp] == i) continue;
                                 const int u = (pp / G) % U, lane = r * G + pp % G;
-                                col[((rec * (U / 4) + u / 4) * SELLW + lane) * 4 + u % 4] = A->ja[k0 + pp] * xsz;
-                                val[((rec * (U / E) + u / E) * SELLW + lane) * E + u % E] = A->a[k0 + pp];
+                                col[((rec * (U / 4) + u / 4) * SELLW + lane) * 4 + u % 4] = place[D->ja[k0 + pp]] * xsz;
+                                val[((rec * (U / E) + u / E) * SELLW + lane) * E + u % E] = D->a[k0 + pp];
                             }
                         }
                     }
                 }
-                t += tmax;
+                t += most;
             }
+        }
     }
-    void *dr = NULL, *dc = NULL, *dv = NULL, *dd = NULL;
-    if (!e) e = upload_ints((int **)&dr, row, 2 * places * R, s->stream);
+    void *dr = NULL, *dc = NULL, *dv = NULL;
+    if (!e) e = upload_ints((int **)&dr, sched, 2 * places, s->stream);
     if (!e) e = upload_ints((int **)&dc, col, recs * U * SELLW, s->stream);
     if (!e) e = upload_real(&dv, val, recs * U * SELLW, s->xt, s->stream);
-    if (!e) e = upload_real(&dd, diag, 2 * recs * R, s->xt, s->stream);
     const int e2 = jxamd_stream_sync(s->stream);
-    o->row = (const int *)dr;
+    o->sched = (const int *)dr;
     o->col = (const unsigned int *)dc;
     o->val = dv;
-    o->diag = dd;
     o->steps = (int)steps;
-    free(row); free(diag); free(col); free(val);
+    free(sched); free(col); free(val);
     return e ? e : e2;
 }
 
 /* Exact sweeps of level l with its vector in LDS, where it fits and where one
- * workgroup is the faster.  Measured: a step of W wavefronts with U entries
- * per lane takes 0.2 + 0.0075 U W us (barrier, gathers, division; the
- * wavefronts' instructions), records beyond the L2 come at some 45 GB/s;
- * k_gs_sweep takes about 2.3 us per dependency level on the whole device. */
+ * workgroup is the faster.  A step of W wavefronts with U entries per lane
+ * takes 0.16 + (0.017 + 0.0064 U) W us (barrier, gathers, division; the
+ * wavefronts' instructions and loads, idle ones too), a record 0.0056 U us
+ * more: fitted to all (G, U, W) on seven levels of 2048 to 20160 rows, within
+ * 13 %; the choice is the measured best or within 10 % of it.  k_gs_sweep takes
+ * about 2.3 us per dependency level on the whole device. */
 static int build_lds(jxamd_solver *s, int l, const jxamd_csr *A)
 {
     dlds *g = &s->Gl[l];
     const int n = A->n, cap = jxamd_gs_lds_rows && jxamd_k_gs_lds ? jxamd_gs_lds_rows(s->xt) : 0;
     if (n < 1 || n > cap || s->vt != s->xt) return 0;
-    int *ord[2] = {NULL, NULL}, *start[2] = {NULL, NULL}, nl[2] = {0, 0}, e = 0;
-    for (int d = 0; d < 2 && !e; d++) {
-        ord[d] = (int *)malloc(sizeof(int) * (size_t)n);
-        e = ord[d] ? lds_levels(A, d ? -1 : 1, ord[d], &start[d], &nl[d]) : JXAMD_ERROR_MEMORY;
-    }
-    if (!e && nl[0] && nl[1]) {
-        double best = 2.3 * nl[0];
+    int *ord = (int *)malloc(sizeof(int) * (size_t)n), *place = (int *)malloc(sizeof(int) * (size_t)n), *start = NULL;
+    double *diag = (double *)calloc(2 * ((size_t)n + JXAMD_LDS_PAD), sizeof(double));
+    int nl = 0, e = !ord || !place || !diag ? JXAMD_ERROR_MEMORY : 0;
+    jxamd_csr D[2];
+    memset(D, 0, sizeof(D));
+    for (int d = 0; d < 2 && !e; d++) e = lds_deps(A, d ? -1 : 1, &D[d]);
+    if (!e) e = lds_levels(&D[0], &D[1], ord, &start, &nl);
+    if (!e && nl) {
+        double best = 2.0 * 2.3 * nl;
         int G = 0, U = 0, W = 0;
         for (int g1 = 1; g1 <= 16; g1 *= 2)
             for (int u1 = 4; u1 <= 8; u1 += 4)
-                for (int w1 = 1; w1 <= 16; w1 *= 2) {
-                    long nrec = 0;
-                    const long steps = lds_steps(A, ord[0], start[0], nl[0], g1, u1, w1, &nrec);
-                    const double bytes = (double)nrec * SELLW * u1 * (4.0 + (double)s->xsz);
-                    const double lane = (0.2 + 0.0075 * u1 * w1) * (double)steps;
-                    const double c = bytes > 2.0e6 && bytes / 45.0e3 > lane ? bytes / 45.0e3 : lane;
+                for (int w1 = 1; w1 <= JXAMD_LDS_WAVES(u1, s->xt); w1 *= 2) {
+                    double c = 0.0;
+                    for (int d = 0; d < 2; d++) {
+                        long nrec = 0;
+                        const long steps = lds_steps(&D[d], ord, start, nl, g1, u1, w1, &nrec);
+                        c += (0.16 + (0.017 + 0.0064 * u1) * w1) * (double)steps + 0.0056 * u1 * (double)nrec;
+                    }
                     if (c < best) { best = c; G = g1; U = u1; W = w1; }
                 }
-        for (int d = 0; d < 2 && !e && W; d++) e = lds_build(s, A, ord[d], start[d], nl[d], G, U, W, &g->sw[d]);
+        if (W) {
+            for (int q = 0; q < n; q++) {
+                /* the diagonal as the kernel holds it, and its reciprocal */
+                const double di = s->xt == JXAMD_T_F64 ? A->a[A->ia[ord[q]]] : (double)(float)A->a[A->ia[ord[q]]];
+                place[ord[q]] = q;
+                diag[2 * q] = di;
+                diag[2 * q + 1] = di != 0.0 ? 1.0 / di : 0.0;
+            }
+            for (int d = 0; d < 2 && !e; d++)
+                e = lds_build(s, &D[d], d ? -1 : 1, ord, place, start, nl, G, U, W, &g->sw[d]);
+            if (!e) e = upload_ints(&g->order, ord, (size_t)n, s->stream);
+            if (!e) e = upload_real(&g->diag, diag, 2 * ((size_t)n + JXAMD_LDS_PAD), s->xt, s->stream);
+            if (!e) e = jxamd_dev_malloc(&g->work, 2 * s->xsz * ((size_t)n + JXAMD_LDS_PAD));
+            const int e2 = jxamd_stream_sync(s->stream);
+            if (!e) e = e2;
+        }
         g->G = G;
         g->U = U;
         g->W = e ? 0 : W;
     }
-    for (int d = 0; d < 2; d++) { free(ord[d]); free(start[d]); }
+    free(ord); free(place); free(start); free(diag);
+    for (int d = 0; d < 2; d++) { free((void *)D[d].ia); free((void *)D[d].ja); free((void *)D[d].a); }
     return e;
 }
 
@@ -2149,9 +2194,9 @@ int jxamd_solver_destroy(jxamd_solver *s)
         dsell_free(&s->Ares[l]); dsell_free(&s->Gf[l]); dsell_free(&s->Gb[l]); dsell_free(&s->Gc[l]);
         for (int d = 0; d < 2; d++) {
             const jxamd_lds_sweep *w = &s->Gl[l].sw[d];
-            jxamd_dev_free((void *)w->row); jxamd_dev_free((void *)w->col);
-            jxamd_dev_free((void *)w->val); jxamd_dev_free((void *)w->diag);
+            jxamd_dev_free((void *)w->sched); jxamd_dev_free((void *)w->col); jxamd_dev_free((void *)w->val);
         }
+        jxamd_dev_free(s->Gl[l].order); jxamd_dev_free(s->Gl[l].diag); jxamd_dev_free(s->Gl[l].work);
         jxamd_dev_free(s->wstep[l]);
         jxamd_dev_free(s->dinvl[l]);
         dsell_free(&s->R[l]); dsell_free(&s->P[l]);
@@ -2238,8 +2283,8 @@ static int hsgs_lds(jxamd_solver *s, int l, const void *f, int fs, void *u, int 
 {
     const dlds *g = &s->Gl[l];
     int pq = prof_begin(s);
-    CK(jxamd_k_gs_lds(g->G, g->U, g->W, s->xt, s->nlev[l], &g->sw[0], &g->sw[1], ncalls, f, fs, uo_zero ? NULL : u, u,
-                      s->stream));
+    CK(jxamd_k_gs_lds(g->G, g->U, g->W, s->xt, s->nlev[l], &g->sw[0], &g->sw[1], g->order, g->diag, ncalls, f, fs,
+                      uo_zero ? NULL : u, u, g->work, s->stream));
     prof_end_level(s, pq, JXAMD_PROF_GS_SWEEP, l, 2.0 * ncalls * g->abytes);
     return 0;
 }
