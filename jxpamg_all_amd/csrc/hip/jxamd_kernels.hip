@@ -945,6 +945,55 @@ k_bhgs_multi(int nsl, int nvs, const int *__restrict__ vorder, const int *__rest
     }
 }
 
+// the forward recurrence over one partition, by one lane: h holds the rows' sums
+// but for the in-partition lower blocks (L, packed by pairs) and takes the new
+// values; len rows from rl in the workgroup's arrays, row ns of the matrix
+template <int B, int LMAX, typename LT, typename DV>
+__device__ __forceinline__ void part_recurrence(int ns, int len, int rl, const LT *L0, const DV *__restrict__ dinv,
+                                                double *h, const double *xold, double w, double omega)
+{
+    const double prod = 1.0 - w * omega;
+    double xnew[LMAX][B];
+#pragma unroll
+    for (int t = 0; t < LMAX; t++) {
+        if (t < len) {
+            double tmp[B];
+#pragma unroll
+            for (int q = 0; q < B; q++) tmp[q] = h[(rl + t) * B + q];
+#pragma unroll
+            for (int u = 0; u < LMAX - 1; u++) {
+                if (u < t) {
+                    const LT *L = L0 + ((t * (t - 1)) / 2 + u) * B * B;
+#pragma unroll
+                    for (int rr = 0; rr < B; rr++)
+#pragma unroll
+                        for (int q = 0; q < B; q++) tmp[rr] -= (double)L[rr * B + q] * xnew[u][q];
+                }
+            }
+            const DV *D = dinv ? dinv + (size_t)(ns + t) * B * B : nullptr;
+#pragma unroll
+            for (int rr = 0; rr < B; rr++) {
+                double o = 0.0;
+                if (D) {
+#pragma unroll
+                    for (int q = 0; q < B; q++) o += (double)D[rr * B + q] * tmp[q];
+                } else {
+                    o = tmp[rr]; // identity diagonal blocks (ABF-decoupled rows)
+                }
+                xnew[t][rr] = prod * xold[(rl + t) * B + rr] + w * o;
+            }
+        } else {
+#pragma unroll
+            for (int q = 0; q < B; q++) xnew[t][q] = 0.0;
+        }
+    }
+#pragma unroll
+    for (int t = 0; t < LMAX; t++)
+        if (t < len)
+#pragma unroll
+            for (int q = 0; q < B; q++) h[(rl + t) * B + q] = xnew[t][q];
+}
+
 // One forward block hybrid SOR sweep as run on nparts ranks (contiguous
 // block-row partitions of at most LMAX rows, first nb % nparts one row
 // longer; par_relax_bsr.c:296-330 and :523-557 with the other ranks'
@@ -956,21 +1005,20 @@ k_bhgs_multi(int nsl, int nvs, const int *__restrict__ vorder, const int *__rest
 // Everything but the x_new terms is row-parallel (phase A, one lane per row
 // over the SpMV layout: SELL-64, all blocks, natural order); the in-partition
 // lower blocks go to LDS and one lane per partition runs the short forward
-// recurrence (phase B).  x_old: xo (B values per row) or, when xo ==
-// nullptr, the prolongated pressure xp (slot pidx, zeros elsewhere; XP
-// double, or float for a stage-1 result in FP32, widened as it is read).
+// recurrence (phase B).  x_old: xo, B values per row (k_bhgs_first takes the
+// first sweep of an application, whose x_old is the prolongated pressure).
 // Blocks are stored as V (double, float, or __half scaled per block row:
 // A_ij = rsc[i] * H_ij), inverted diagonal blocks as DV (dinv == nullptr:
 // every diagonal block is the identity, as after ABF decoupling, and none
 // is read); arithmetic in double.  PU slots per batch.
-template <int B, int LMAX, typename V, typename DV, int PU, typename XP>
+template <int B, int LMAX, typename V, typename DV, int PU>
 __global__ void __launch_bounds__(256) k_bhgs_part(int nb, int nparts, int cpb, const int *__restrict__ sptr,
                                                    const int *__restrict__ pptr,
                                                    const int *__restrict__ col, const V *__restrict__ val,
                                                    const float *__restrict__ rsc, const DV *__restrict__ dinv,
                                                    const double *__restrict__ rhs,
-                                                   const double *__restrict__ xo, const XP *__restrict__ xp,
-                                                   int pidx, double *__restrict__ xn, double w, double omega)
+                                                   const double *__restrict__ xo, double *__restrict__ xn, double w,
+                                                   double omega)
 {
     constexpr int NL = LMAX * (LMAX - 1) / 2; // strictly lower pairs of a partition
     constexpr int LST = NL * B * B + 1;       // odd stride between partitions
@@ -1037,7 +1085,7 @@ __global__ void __launch_bounds__(256) k_bhgs_part(int nb, int nparts, int cpb, 
                 const int j = jj[u];
 #pragma unroll
                 for (int q = 0; q < B; q++)
-                    xj[u][q] = j == i ? 0.0 : (xo ? xo[(size_t)j * B + q] : (q == pidx ? (double)xp[j] : 0.0));
+                    xj[u][q] = j == i ? 0.0 : xo[(size_t)j * B + q];
             }
 #pragma unroll
             for (int u = 0; u < PU; u++) {
@@ -1071,56 +1119,132 @@ __global__ void __launch_bounds__(256) k_bhgs_part(int nb, int nparts, int cpb, 
 #pragma unroll
         for (int q = 0; q < B; q++) {
             h[r * B + q] = omega * res[q] + res0[q] + (1.0 - omega) * res2[q];
-            xold[r * B + q] = xo ? xo[(size_t)i * B + q] : (q == pidx ? (double)xp[i] : 0.0);
+            xold[r * B + q] = xo[(size_t)i * B + q];
         }
     }
     __syncthreads();
     const int c = c0 + (int)threadIdx.x;
     if (c < c1) {
         const int ns = c < rest ? c * (size + 1) : c * size + rest;
+        part_recurrence<B, LMAX>(ns, c < rest ? size + 1 : size, ns - row0, Lb + (size_t)(c - c0) * LST, dinv, h, xold, w,
+                                 omega);
+    }
+    __syncthreads();
+    if (i < row1)
+#pragma unroll
+        for (int q = 0; q < B; q++) xn[(size_t)i * B + q] = h[r * B + q];
+}
+
+// The sweep from the prolongated pressure: x_old is xp in slot pidx and zero
+// elsewhere (XP double, or float for a stage-1 result in FP32, widened as it is
+// read), so a coupling outside the partition, or above the row, needs only
+// column pidx of its block; the other values are read for the in-partition
+// lower blocks alone.  Layouts and results as k_bhgs_part.  Measured, with the
+// general kernel and now: 60x220x85 3x3 118 and 66 us (FP64 blocks), 50 and
+// 40 us (FP16); 61x47x53 4x4 FP64 50 and 27 us; 41x97x37 3x3 FP32 18 and 12 us.
+template <int B, int LMAX, typename V, typename DV, int PU, typename XP>
+__global__ void __launch_bounds__(256) k_bhgs_first(int nb, int nparts, int cpb, const int *__restrict__ sptr,
+                                                    const int *__restrict__ pptr, const int *__restrict__ col,
+                                                    const V *__restrict__ val, const float *__restrict__ rsc,
+                                                    const DV *__restrict__ dinv, const double *__restrict__ rhs,
+                                                    const XP *__restrict__ xp, int pidx, double *__restrict__ xn,
+                                                    double w, double omega)
+{
+    constexpr int LST = (LMAX * (LMAX - 1) / 2) * B * B + 1;
+    constexpr bool HALF = constexpr_is_half<V>::value; // slot pairs in 32-bit words, as in k_bhgs_part
+    typedef typename lds_block<V>::T LT;
+    extern __shared__ __align__(16) unsigned char smraw[];
+    double *sm = reinterpret_cast<double *>(smraw);
+    double *h = sm, *xold = sm + 256 * B;
+    LT *Lb = reinterpret_cast<LT *>(sm + 2 * 256 * B);
+    const int size = nb / nparts, rest = nb - size * nparts;
+    const int c0 = xcd_tile(blockIdx.x, gridDim.x) * cpb;
+    const int c1 = min(c0 + cpb, nparts);
+    const int row0 = c0 < rest ? c0 * (size + 1) : c0 * size + rest;
+    const int row1 = c1 < rest ? c1 * (size + 1) : c1 * size + rest;
+    for (int e = threadIdx.x; e < cpb * LST; e += blockDim.x) Lb[e] = (LT)0;
+    __syncthreads();
+    const int r = threadIdx.x;
+    const int i = row0 + r;
+    if (i < row1) {
+        const int big = rest * (size + 1);
+        const int c = i < big ? i / (size + 1) : rest + (i - big) / size;
+        const int ns = c < rest ? c * (size + 1) : c * size + rest;
         const int len = c < rest ? size + 1 : size;
-        const int rl = ns - row0;
-        const LT *Lc = Lb + (size_t)(c - c0) * LST;
-        const double prod = 1.0 - w * omega;
-        double xnew[LMAX][B];
+        const int ti = i - ns;
+        double res[B], res0[B], res2[B];
 #pragma unroll
-        for (int t = 0; t < LMAX; t++) {
-            if (t < len) {
-                double tmp[B];
+        for (int q = 0; q < B; q++) {
+            res[q] = rhs[(size_t)i * B + q];
+            res0[q] = 0.0;
+            res2[q] = 0.0;
+        }
+        const double xi = (double)xp[i];
+        const int s = i / WAVE, lane = i % WAVE;
+        const double sc = row_scaled<V>::value ? (double)rsc[i] : 1.0;
+        const int ks = sptr[s], k1 = sptr[s + 1], ps = HALF ? pptr[s] : 0;
+        // value e of the block in slot k of the lane, or of the slot's pair
+        auto word = [&](int k, int e) {
+            if constexpr (HALF)
+                return reinterpret_cast<const __half2 *>(val)[((size_t)(ps + (k - ks) / 2) * B * B + e) * WAVE + lane];
+            else return ldnt(val + ((size_t)k * B * B + e) * WAVE + lane);
+        };
+        for (int k = ks; k < k1; k += PU) {
+            int jj[PU];
+            double xj[PU];
+            decltype(word(0, 0)) pc[HALF ? PU / 2 : PU][B];
 #pragma unroll
-                for (int q = 0; q < B; q++) tmp[q] = h[(rl + t) * B + q];
+            for (int u = 0; u < PU; u++) jj[u] = k + u < k1 ? col[(size_t)(k + u) * WAVE + lane] : i;
 #pragma unroll
-                for (int u = 0; u < LMAX - 1; u++) {
-                    if (u < t) {
-                        const LT *L = Lc + ((t * (t - 1)) / 2 + u) * B * B;
+            for (int u = 0; u < PU; u += HALF ? 2 : 1)
 #pragma unroll
-                        for (int rr = 0; rr < B; rr++)
+                for (int rr = 0; rr < B; rr++) pc[HALF ? u / 2 : u][rr] = word(k + u < k1 ? k + u : ks, rr * B + pidx);
 #pragma unroll
-                            for (int q = 0; q < B; q++) tmp[rr] -= (double)L[rr * B + q] * xnew[u][q];
-                    }
+            for (int u = 0; u < PU; u++) xj[u] = jj[u] == i ? 0.0 : (double)xp[jj[u]];
+#pragma unroll
+            for (int u = 0; u < PU; u++) {
+                const int j = jj[u];
+                if (j < ns || j >= i) continue; // in-partition lower blocks
+                LT *L = Lb + (size_t)(c - c0) * LST + ((ti * (ti - 1)) / 2 + (j - ns)) * B * B;
+#pragma unroll
+                for (int e = 0; e < B * B; e++) {
+                    double v;
+                    if constexpr (HALF) v = (double)(u & 1 ? __high2float(word(k + u, e)) : __low2float(word(k + u, e)));
+                    else v = (double)word(k + u, e);
+                    L[e] = (LT)(sc * v);
                 }
-                const DV *D = dinv ? dinv + (size_t)(ns + t) * B * B : nullptr;
+            }
+#pragma unroll
+            for (int u = 0; u < PU; u++) {
+                const int j = jj[u];
+                if (j == i) continue; // the diagonal block, padding, or past the slice
+                const bool in = j >= ns && j < ns + len;
 #pragma unroll
                 for (int rr = 0; rr < B; rr++) {
-                    double o = 0.0;
-                    if (D) {
-#pragma unroll
-                        for (int q = 0; q < B; q++) o += (double)D[rr * B + q] * tmp[q];
-                    } else {
-                        o = tmp[rr]; // identity diagonal blocks (ABF-decoupled rows)
+                    double v;
+                    if constexpr (HALF) v = (double)(u & 1 ? __high2float(pc[u / 2][rr]) : __low2float(pc[u / 2][rr]));
+                    else v = (double)pc[u][rr];
+                    const double acc = v * xj[u] * sc;
+                    if (!in) res[rr] -= acc;
+                    else {
+                        res2[rr] += acc;
+                        if (j > i) res0[rr] -= acc;
                     }
-                    xnew[t][rr] = prod * xold[(rl + t) * B + rr] + w * o;
                 }
-            } else {
-#pragma unroll
-                for (int q = 0; q < B; q++) xnew[t][q] = 0.0;
             }
         }
 #pragma unroll
-        for (int t = 0; t < LMAX; t++)
-            if (t < len)
-#pragma unroll
-                for (int q = 0; q < B; q++) h[(rl + t) * B + q] = xnew[t][q];
+        for (int q = 0; q < B; q++) {
+            h[r * B + q] = omega * res[q] + res0[q] + (1.0 - omega) * res2[q];
+            xold[r * B + q] = q == pidx ? xi : 0.0;
+        }
+    }
+    __syncthreads();
+    const int c = c0 + (int)threadIdx.x;
+    if (c < c1) {
+        const int ns = c < rest ? c * (size + 1) : c * size + rest;
+        part_recurrence<B, LMAX>(ns, c < rest ? size + 1 : size, ns - row0, Lb + (size_t)(c - c0) * LST, dinv, h, xold, w,
+                                 omega);
     }
     __syncthreads();
     if (i < row1)
@@ -2291,31 +2415,29 @@ int jxamd_k_bhgs_part(int b, int vt, int nb, int nparts, const int *sptr, const 
     // FP32 4, FP16 2 (66 -> 52 us against 4: 75 instead of 109 VGPRs, six
     // waves per SIMD instead of four)
     constexpr int PU64 = 6, PU32 = 4, PU16 = 2;
+    constexpr int PUF = 6; // k_bhgs_first: the stencil's off-diagonals at once
 #define LAUNCH_PART(BS, LM)                                                                                            \
-    do {                                                                                                               \
-        if (xp_f32) LAUNCH_PART_X(BS, LM, float);                                                                     \
-        else LAUNCH_PART_X(BS, LM, double);                                                                            \
-    } while (0)
-#define LAUNCH_PART_X(BS, LM, XT)                                                                                      \
     do {                                                                                                               \
         const int cpb = 256 / LM;                                                                                      \
         const int grid = (nparts + cpb - 1) / cpb;                                                                     \
         const size_t lb = (size_t)cpb * ((LM * (LM - 1) / 2) * BS * BS + 1);                                          \
         const size_t lds = sizeof(double) * 2 * 256 * BS + (vt == JXAMD_T_F64 ? sizeof(double) : sizeof(float)) * lb; \
-        if (vt == JXAMD_T_F64)                                                                                        \
-            k_bhgs_part<BS, LM, double, double, PU64, XT><<<grid, 256, lds, st>>>(                                     \
-                nb, nparts, cpb, sptr, pptr, col, (const double *)val, rsc, (const double *)dinv, rhs, xo,             \
-                (const XT *)xp,                                                                                        \
-                pidx, xn, w, omega);                                                                                   \
-        else if (vt == JXAMD_T_F32)                                                                                    \
-            k_bhgs_part<BS, LM, float, float, PU32, XT><<<grid, 256, lds, st>>>(                                       \
-                nb, nparts, cpb, sptr, pptr, col, (const float *)val, rsc, (const float *)dinv, rhs, xo,               \
-                (const XT *)xp,                                                                                        \
+        if (vt == JXAMD_T_F64) LAUNCH_PART_V(BS, LM, double, double, PU64);                                           \
+        else if (vt == JXAMD_T_F32) LAUNCH_PART_V(BS, LM, float, float, PU32);                                        \
+        else LAUNCH_PART_V(BS, LM, __half, float, PU16);                                                               \
+    } while (0)
+#define LAUNCH_PART_V(BS, LM, VT, DT, PU)                                                                              \
+    do {                                                                                                               \
+        if (xo)                                                                                                        \
+            k_bhgs_part<BS, LM, VT, DT, PU><<<grid, 256, lds, st>>>(nb, nparts, cpb, sptr, pptr, col, (const VT *)val, \
+                                                                    rsc, (const DT *)dinv, rhs, xo, xn, w, omega);     \
+        else if (xp_f32)                                                                                               \
+            k_bhgs_first<BS, LM, VT, DT, PUF, float><<<grid, 256, lds, st>>>(                                          \
+                nb, nparts, cpb, sptr, pptr, col, (const VT *)val, rsc, (const DT *)dinv, rhs, (const float *)xp,      \
                 pidx, xn, w, omega);                                                                                   \
         else                                                                                                           \
-            k_bhgs_part<BS, LM, __half, float, PU16, XT><<<grid, 256, lds, st>>>(                                      \
-                nb, nparts, cpb, sptr, pptr, col, (const __half *)val, rsc, (const float *)dinv, rhs, xo,              \
-                (const XT *)xp,                                                                                        \
+            k_bhgs_first<BS, LM, VT, DT, PUF, double><<<grid, 256, lds, st>>>(                                         \
+                nb, nparts, cpb, sptr, pptr, col, (const VT *)val, rsc, (const DT *)dinv, rhs, (const double *)xp,     \
                 pidx, xn, w, omega);                                                                                   \
     } while (0)
 #define PART_B(BS)                                                                                                     \
@@ -2332,7 +2454,7 @@ int jxamd_k_bhgs_part(int b, int vt, int nb, int nparts, const int *sptr, const 
     }
 #undef PART_B
 #undef LAUNCH_PART
-#undef LAUNCH_PART_X
+#undef LAUNCH_PART_V
     return chk(hipGetLastError());
 }
 

@@ -64,6 +64,7 @@ typedef struct {
     double spmv_bytes, sweep_bytes; /* algorithmic bytes: y = A x, one fused one-rank block-HGS sweep */
     int unit_diag;             /* every diagonal block is exactly the identity: the partitioned sweeps skip Dinv */
     double part_bytes, part_bytes32; /* algorithmic bytes of one partitioned sweep (FP64, narrow blocks) */
+    double first_less;               /* block values the sweep from the prolongated pressure does not need */
 } dbsr;
 
 /* one BILU(0) triangle on the device: level-ordered block SELL of the
@@ -1317,6 +1318,18 @@ static int build_bsr(jxamd_solver *s, const jxamd_bsr *A)
             d->part_bytes = common + nblk * 8.0 * bb + (d->unit_diag ? 0.0 : 8.0 * nb * bb);
             d->part_bytes32 = common + nblk * sv * bb + (d->unit_diag ? 0.0 : 4.0 * nb * bb) +
                               (s->prm.stage2_precision == 2 ? 4.0 * nb : 0.0);
+            /* the first sweep (k_bhgs_first): one column of every block but
+             * those below the row inside its partition, no vector but xp */
+            long whole = 0;
+            if (s->prm.stage2_chunk > 0) {
+                const int parts = (nb + s->prm.stage2_chunk - 1) / s->prm.stage2_chunk, size = nb / parts;
+                const int rest = nb - size * parts, big = rest * (size + 1);
+                for (int i = 0; i < nb; i++) {
+                    const int ns = i < big ? i / (size + 1) * (size + 1) : big + (i - big) / size * size;
+                    for (int k = A->ia[i] + 1; k < A->ia[i + 1]; k++) whole += A->ja[k] >= ns && A->ja[k] < i;
+                }
+            }
+            d->first_less = ((double)(A->nnzb - nb) - (double)whole) * (bb - b);
         }
         /* columns as positions: ~pos for lower neighbours, the own position for padding */
         {
@@ -2526,7 +2539,8 @@ static int cpr_apply(jxamd_solver *s, const double *r, double *x)
                                  d->unit_diag ? NULL : (nar ? d->dinv32 : (const void *)d->dinv), r, src,
                                  xp_f32 ? s->U[0] : (const void *)xp, xp_f32, pi, dst, s->prm.stage2_weight,
                                  s->prm.stage2_omega, s->stream));
-            prof_end(s, pq, JXAMD_PROF_BHGS_SWEEP, nar ? d->part_bytes32 : d->part_bytes);
+            const double less = src ? 0.0 : d->first_less * (double)type_size(stage2_vt(nar)) + 8.0 * (s->N - s->nb);
+            prof_end(s, pq, JXAMD_PROF_BHGS_SWEEP, (nar ? d->part_bytes32 : d->part_bytes) - less);
             src = dst;
             dst = (dst == x) ? s->xtmp : x;
         }
