@@ -141,6 +141,12 @@ int jxamd_k_gs_chunk_lds(int vt, int xt, int n, int nchunks, const int *sptr, co
 int jxamd_k_gs_chunk(int vt, int xt, int n, int nchunks, const int *wstep, const int *sptr, const int *col,
                      const void *val, const float *rsc, const void *diag, const void *f, int fs, const void *uo,
                      void *un, void *stream);
+/* the same from a zero guess, on the chunks' own couplings alone (blk: row t to
+ * row q of chunk c, q counted without t, at ((c / 64) L (L - 1) + t (L - 1) +
+ * q) 64 + c % 64); L = 2, 4 or 8, at least the longest chunk; a device layer
+ * may leave it undefined */
+int jxamd_k_gs_chunk_zero(int L, int xt, int n, int nchunks, const void *blk, const void *diag, const void *f, int fs,
+                          void *un, void *stream) __attribute__((weak));
 /* row-group variants (G = 4, 8, 16 or 32 lanes per row): SpMV and polynomial
  * step over the SELL-G layout (64/G rows per slice; sptr: slot-row offsets
  * per slice), the chunked smoother over plain CSR */

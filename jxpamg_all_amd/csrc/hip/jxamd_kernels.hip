@@ -1591,6 +1591,54 @@ __global__ void __launch_bounds__(256) k_poly_step_grp(int n, const int *__restr
     un[row] = e.u + omega * e.d * r;
 }
 
+// The chunked relax-6 call from a zero guess: couplings that leave a chunk meet
+// zeros, so only the chunks' own couplings are read, from blk: entry
+// e = t (LMAX - 1) + q (q counted without t) of chunk c, the coupling of its row
+// t to its row q, at ((c / 64) LMAX (LMAX - 1) + e) 64 + c % 64.  One lane per
+// chunk, the recurrence of k_gs_chunk_lds (the forward sweep without the rows
+// that are still zero).  Measured, with the general kernels and now: levels of
+// the 60x220x85 system, FP64, 1122000 rows of 7 25.5 and 18.3 us, 560800 of 24
+// 45 and 8.0, 136100 of 105 50 and 5.0; 61x47x53, 151900 of 7 7.8 and 4.9 us.
+template <int LMAX, typename X>
+__global__ void __launch_bounds__(256) k_gs_chunk_zero(int n, int nchunks, const X *__restrict__ blk,
+                                                       const X *__restrict__ diag, const X *__restrict__ f, int fs,
+                                                       X *__restrict__ un)
+{
+    constexpr int NE = LMAX * (LMAX - 1);
+    const int c = xcd_tile(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
+    if (c >= nchunks) return;
+    const int size = n / nchunks, rest = n - size * nchunks;
+    const int ns = c < rest ? c * (size + 1) : c * size + rest, len = c < rest ? size + 1 : size;
+    const X *bc = blk + (size_t)(c / WAVE) * NE * WAVE + c % WAVE;
+    X B[NE], u[LMAX], g[LMAX], d[LMAX];
+#pragma unroll
+    for (int t = 0; t < LMAX; t++) {
+        const int i = ns + min(t, len - 1);
+        g[t] = f[(size_t)i * fs];
+        d[t] = diag[i];
+        u[t] = 0;
+    }
+#pragma unroll
+    for (int e = 0; e < NE; e++) B[e] = bc[(size_t)e * WAVE];
+#pragma unroll
+    for (int pass = 0; pass < 2; pass++) {
+#pragma unroll
+        for (int tt = 0; tt < LMAX; tt++) {
+            const int t = pass == 0 ? tt : LMAX - 1 - tt;
+            if (t < len && d[t] != (X)0) {
+                X x = g[t];
+#pragma unroll
+                for (int q = 0; q < LMAX; q++)
+                    if (q != t && q < len && (pass > 0 || q < t)) x -= B[t * (LMAX - 1) + (q < t ? q : q - 1)] * u[q];
+                u[t] = x / d[t];
+            }
+        }
+    }
+#pragma unroll
+    for (int t = 0; t < LMAX; t++)
+        if (t < len) un[ns + t] = u[t];
+}
+
 // chunked hybrid SSOR (as k_gs_chunk_lds) with phase A done by row groups
 // over plain CSR (ia, ja, val; diagonal first, kept apart in diag): a block
 // covers whole chunks, so its rows start anywhere in a slice of any layout;
@@ -2620,6 +2668,32 @@ int jxamd_k_gs_sweep_grp(int G, int vt, int xt, int nsl, const int *perm, const 
                                   (const X_ *)uo, (X_ *)un, dep_ptr, dep_list, sflag, epoch, dir, ticket, *base,
                                   err))));
     *base += (unsigned long long)nsl + (unsigned long long)grid * 4;
+    return chk(hipGetLastError());
+}
+
+int jxamd_k_gs_chunk_zero(int L, int xt, int n, int nchunks, const void *blk, const void *diag, const void *f, int fs,
+                          void *un, void *stream)
+{
+    if (n == 0 || nchunks < 1) return 0;
+    if (jxamd_gs_chunk_lds_rows(n, nchunks) > L) return JXAMD_ERROR_ARG;
+    const int grid = (nchunks + 255) / 256;
+    hipStream_t st = (hipStream_t)stream;
+#define LAUNCH_CZ(LM)                                                                                                  \
+    do {                                                                                                               \
+        if (xt == JXAMD_T_F64)                                                                                         \
+            k_gs_chunk_zero<LM, double><<<grid, 256, 0, st>>>(n, nchunks, (const double *)blk, (const double *)diag,   \
+                                                              (const double *)f, fs, (double *)un);                    \
+        else                                                                                                           \
+            k_gs_chunk_zero<LM, float><<<grid, 256, 0, st>>>(n, nchunks, (const float *)blk, (const float *)diag,      \
+                                                             (const float *)f, fs, (float *)un);                       \
+    } while (0)
+    switch (L) {
+    case 2: LAUNCH_CZ(2); break;
+    case 4: LAUNCH_CZ(4); break;
+    case 8: LAUNCH_CZ(8); break;
+    default: return JXAMD_ERROR_ARG;
+    }
+#undef LAUNCH_CZ
     return chk(hipGetLastError());
 }
 

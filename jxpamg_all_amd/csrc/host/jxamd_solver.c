@@ -117,6 +117,9 @@ struct jxamd_solver_s {
     dsell Ares[JXAMD_MAX_LEVELS], Gf[JXAMD_MAX_LEVELS], Gb[JXAMD_MAX_LEVELS];
     dsell Gc[JXAMD_MAX_LEVELS]; /* threaded relax-6 layout (chunked mode) */
     dlds Gl[JXAMD_MAX_LEVELS];  /* exact sweeps with the vector in LDS (Gf, Gb are then not built) */
+    int zeroL[JXAMD_MAX_LEVELS];  /* chunked mode: rows a block of Gz holds (0: no Gz) */
+    void *Gz[JXAMD_MAX_LEVELS];   /* couplings inside the chunks, for calls from a zero guess */
+    double zbytes[JXAMD_MAX_LEVELS];
     int *wstep[JXAMD_MAX_LEVELS];
     int nchunks[JXAMD_MAX_LEVELS]; /* 0: sequential sweeps on this level */
     dsell R[JXAMD_MAX_LEVELS], P[JXAMD_MAX_LEVELS];
@@ -1927,6 +1930,39 @@ static int build_lds(jxamd_solver *s, int l, const jxamd_csr *A)
     return e;
 }
 
+/* The couplings inside the chunks of level l (T chunks) for relax-6 calls from
+ * a zero guess (jxamd_k_gs_chunk_zero), where they are at most half of the
+ * stored entries: blocks of L rows hold L - 1 values per row against a mean
+ * row's entries and their columns. */
+static int build_chunk_zero(jxamd_solver *s, int l, const jxamd_csr *A, int T)
+{
+    const int n = A->n, longest = jxamd_gs_chunk_lds_rows(n, T);
+    int L = 2;
+    while (L < longest) L *= 2;
+    if (!jxamd_k_gs_chunk_zero || s->vt != s->xt || L > 8 || 2.0 * (L - 1) * n > (double)A->ia[n]) return 0;
+    const int size = n / T, rest = n - size * T, NE = L * (L - 1);
+    const size_t nv = (size_t)((T + SELLW - 1) / SELLW) * NE * SELLW;
+    double *v = (double *)calloc(nv, sizeof(double));
+    if (!v) return JXAMD_ERROR_MEMORY;
+#pragma omp parallel for schedule(static) if (n > 20000)
+    for (int c = 0; c < T; c++) {
+        const int ns = c < rest ? c * (size + 1) : c * size + rest, len = c < rest ? size + 1 : size;
+        double *vc = v + (size_t)(c / SELLW) * NE * SELLW + c % SELLW;
+        for (int t = 0; t < len; t++)
+            for (int k = A->ia[ns + t] + 1; k < A->ia[ns + t + 1]; k++) {
+                const int q = A->ja[k] - ns;
+                if (q < 0 || q >= len || q == t) continue;
+                vc[(size_t)(t * (L - 1) + (q < t ? q : q - 1)) * SELLW] += A->a[k];
+            }
+    }
+    int e = upload_real(&s->Gz[l], v, nv, s->xt, s->stream);
+    const int e2 = jxamd_stream_sync(s->stream);
+    free(v);
+    s->zeroL[l] = L;
+    s->zbytes[l] = (double)s->xsz * ((double)nv + 3.0 * n);
+    return e ? e : e2;
+}
+
 static int build_level_mats(jxamd_solver *s, int l, const jxamd_hierarchy *H, const jxamd_csr *A)
 {
     const int n = A->n;
@@ -1969,6 +2005,7 @@ static int build_level_mats(jxamd_solver *s, int l, const jxamd_hierarchy *H, co
         s->wstep[l] = NULL;
         /* matrix once, f + entry values + results */
         s->Gc[l].abytes = level_bytes(&s->Gc[l], A->ia[n], n, 3.0);
+        CK(build_chunk_zero(s, l, A, T));
     } else if (T > 1 && (l < s->L - 1 || s->L == 1)) {
         /* long chunks: wave w holds chunks 64w..64w+63; slice wstep[w]+t
          * holds row ns(c)+t of each chunk c of the wave */
@@ -2211,6 +2248,7 @@ int jxamd_solver_destroy(jxamd_solver *s)
         }
         jxamd_dev_free(s->Gl[l].order); jxamd_dev_free(s->Gl[l].diag); jxamd_dev_free(s->Gl[l].work);
         jxamd_dev_free(s->wstep[l]);
+        jxamd_dev_free(s->Gz[l]);
         jxamd_dev_free(s->dinvl[l]);
         dsell_free(&s->R[l]); dsell_free(&s->P[l]);
         jxamd_dev_free(s->F[l]); jxamd_dev_free(s->U[l]); jxamd_dev_free(s->T[l]); jxamd_dev_free(s->Vt[l]);
@@ -2307,6 +2345,12 @@ static int hsgs_chunk(jxamd_solver *s, int l, const void *f, int fs, const void 
 {
     dsell *g = &s->Gc[l];
     int pq = prof_begin(s);
+    if (!uo && s->zeroL[l]) {
+        CK(jxamd_k_gs_chunk_zero(s->zeroL[l], s->xt, s->nlev[l], s->nchunks[l], s->Gz[l], g->diag, f, fs, un,
+                                 s->stream));
+        prof_end_level(s, pq, JXAMD_PROF_GS_SWEEP, l, s->zbytes[l]);
+        return 0;
+    }
     if (s->wstep[l])
         CK(jxamd_k_gs_chunk(g->vt, g->xt, s->nlev[l], s->nchunks[l], s->wstep[l], g->sptr, g->col, g->val, g->rsc,
                             g->diag, f, fs, uo, un, s->stream));
