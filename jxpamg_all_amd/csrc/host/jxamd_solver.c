@@ -416,6 +416,12 @@ static int build_vorder(const hsched *sc, const int *nb_ptr, const int *nb_list,
     return 0;
 }
 
+/* rows from which the host lays a matrix out on all cores; below, the threads'
+ * start takes as long as the loop.  Creating a solver from a hierarchy, with
+ * one core per layout and with sixteen: 60x220x85 1030 and 418 ms, 61x47x53
+ * 4x4 220 and 99 ms. */
+#define LAYOUT_OMP 20000
+
 /* Scalar SELL-64 on the host.  Rows in the order given by perm (identity if
  * NULL).  offdiag: drop the first (diagonal) entry of every row into diag[].
  * pad_self: pad with the row's own index (square smoother matrices), else 0. */
@@ -463,6 +469,7 @@ static int hsell_build(hsell *h, int n, const int *ia, const int *ja, const doub
     h->col = (int *)malloc(sizeof(int) * (size_t)(total > 0 ? total : 1) * SELLW);
     h->val = (double *)malloc(sizeof(double) * (size_t)(total > 0 ? total : 1) * SELLW);
     if (!h->col || !h->val) return JXAMD_ERROR_MEMORY;
+#pragma omp parallel for schedule(static) if (n > LAYOUT_OMP)
     for (int s = 0; s < h->nsl; s++) {
         int k0 = h->sptr[s], w = h->sptr[s + 1] - k0;
         for (int l = 0; l < SELLW; l++) {
@@ -519,8 +526,10 @@ static int pack16_slices(const int *col, const double *val, const int *sp, int n
     const size_t rows = (size_t)w[nsl] + PK16_PAD;
     int32_t *o = (int32_t *)calloc(rows * SELLW, sizeof(int32_t));
     if (!o) { free(w); return 0; }
+    int bad = 0;
+#pragma omp parallel for schedule(static) reduction(| : bad) if (n > LAYOUT_OMP)
     for (int q = 0; q < nsl; q++)
-        for (int k = sp[q]; k < sp[q + 1]; k++)
+        for (int k = sp[q]; k < sp[q + 1] && !bad; k++)
             for (int ln = 0; ln < SELLW; ln++) {
                 const size_t e = (size_t)k * SELLW + ln;
                 const int row = q * R + ln / G;
@@ -528,12 +537,13 @@ static int pack16_slices(const int *col, const double *val, const int *sp, int n
                 if (row >= n) off = (long)(n - 1) - row;
                 else if (val[e] == 0.0) off = 0;
                 else off = (long)col[e] - row;
-                if (off < -32768 || off > 32767) { free(o); free(w); return 0; }
+                if (off < -32768 || off > 32767) { bad = 1; break; }
                 const int t = k - sp[q];
                 const size_t we = ((size_t)w[q] + t / 2) * SELLW + ln;
                 const uint32_t h = (uint32_t)(uint16_t)(int16_t)off;
                 o[we] = (int32_t)((uint32_t)o[we] | (t % 2 ? h << 16 : h));
             }
+    if (bad) { free(o); free(w); return 0; }
     *words = o;
     *wp = w;
     *nw = rows;
@@ -551,6 +561,7 @@ static int upload_pk16(dsell *d, const int *sp, int nsl, const int32_t *o, const
     if (h16) {
         uint16_t *pv = (uint16_t *)calloc(rows * SELLW * 2, sizeof(uint16_t));
         if (!pv) return JXAMD_ERROR_MEMORY;
+#pragma omp parallel for schedule(static) if (nsl > LAYOUT_OMP / SELLW)
         for (int q = 0; q < nsl; q++)
             for (int k = sp[q]; k < sp[q + 1]; k++) {
                 const int t = k - sp[q];
@@ -661,11 +672,13 @@ static int dsell_upload(dsell *d, const hsell *h, int ncols, void *st, const hsc
         float *sc = NULL;
         if (!tmp) return JXAMD_ERROR_MEMORY;
         if (vt == JXAMD_T_F32) {
+#pragma omp parallel for schedule(static) if (h->n > LAYOUT_OMP)
             for (size_t e = 0; e < slots; e++) ((float *)tmp)[e] = (float)h->val[e];
         } else {
             const size_t npos = (size_t)h->nsl * SELLW;
             sc = (float *)malloc(sizeof(float) * (npos ? npos : 1));
             if (!sc) { free(tmp); return JXAMD_ERROR_MEMORY; }
+#pragma omp parallel for schedule(static) if (h->n > LAYOUT_OMP)
             for (int q = 0; q < h->nsl; q++)
                 for (int l = 0; l < SELLW; l++) {
                     double mx = 0.0;
@@ -790,12 +803,14 @@ static int dsellg_upload(dsell *d, int n, int ncols, const int *ia, const int *j
     double *vl = (double *)calloc(tot ? tot : 1, sizeof(double));
     float *sc = vt == JXAMD_T_F16 ? (float *)malloc(sizeof(float) * (n > 0 ? n : 1)) : NULL;
     if (!cl || !vl || (vt == JXAMD_T_F16 && !sc)) { free(sp); free(cl); free(vl); free(sc); return JXAMD_ERROR_MEMORY; }
+#pragma omp parallel for schedule(static) if (n > LAYOUT_OMP)
     for (int q = 0; q < nsl; q++)
         for (int u = sp[q]; u < sp[q + 1]; u++)
             for (int ln = 0; ln < SELLW; ln++) {
                 const int i = q * R + ln / G;
                 cl[(size_t)u * SELLW + ln] = (i < n && i < ncols) ? i : 0;
             }
+#pragma omp parallel for schedule(static) if (n > LAYOUT_OMP)
     for (int i = 0; i < n; i++) {
         const int q = i / R, lr = i % R;
         double scale = 1.0;
@@ -825,10 +840,13 @@ static int dsellg_upload(dsell *d, int n, int ncols, const int *ia, const int *j
     if (!rc && vt != JXAMD_T_F64) {
         tmp = malloc(type_size(vt) * (tot ? tot : 1));
         if (!tmp) rc = JXAMD_ERROR_MEMORY;
-        else if (vt == JXAMD_T_F32)
+        else if (vt == JXAMD_T_F32) {
+#pragma omp parallel for schedule(static) if (n > LAYOUT_OMP)
             for (size_t k = 0; k < tot; k++) ((float *)tmp)[k] = (float)vl[k];
-        else
+        } else {
+#pragma omp parallel for schedule(static) if (n > LAYOUT_OMP)
             for (size_t k = 0; k < tot; k++) ((uint16_t *)tmp)[k] = half_bits((float)vl[k]);
+        }
     }
     if (!rc) rc = jxamd_h2d(d->val, tmp ? tmp : (void *)vl, type_size(vt) * tot, st);
     if (!rc && sc) {
@@ -871,10 +889,12 @@ static int dcsr_upload(dsell *d, int n, int ncols, const int *ia, const int *ja,
         float *sc = NULL;
         if (!tmp) return JXAMD_ERROR_MEMORY;
         if (vt == JXAMD_T_F32) {
+#pragma omp parallel for schedule(static) if (n > LAYOUT_OMP)
             for (size_t k = 0; k < nnz; k++) ((float *)tmp)[k] = (float)a[k];
         } else {
             sc = (float *)malloc(sizeof(float) * (n > 0 ? n : 1));
             if (!sc) { free(tmp); return JXAMD_ERROR_MEMORY; }
+#pragma omp parallel for schedule(static) if (n > LAYOUT_OMP)
             for (int i = 0; i < n; i++) {
                 double mx = 0.0;
                 const int k0 = ia[i + 1] - ia[i] > 1 ? ia[i] + 1 : ia[i];
@@ -1146,6 +1166,7 @@ static int upload_real(void **dst, const double *src, size_t n, int vt, void *st
     if (vt == JXAMD_T_F64) return jxamd_h2d(*dst, src, sizeof(double) * n, st);
     float *t = (float *)malloc(sizeof(float) * (n ? n : 1));
     if (!t) return JXAMD_ERROR_MEMORY;
+#pragma omp parallel for schedule(static) if (n > LAYOUT_OMP)
     for (size_t k = 0; k < n; k++) t[k] = (float)src[k];
     int rc = jxamd_h2d(*dst, t, sizeof(float) * n, st);
     if (!rc) rc = jxamd_stream_sync(st);
@@ -1244,6 +1265,7 @@ static int build_bsr(jxamd_solver *s, const jxamd_bsr *A)
         size_t slots = (size_t)(h.nsl ? h.sptr[h.nsl] : 0);
         double *v = (double *)calloc(slots * bb * SELLW + 1, sizeof(double));
         if (!v) { hsell_free(&h); return JXAMD_ERROR_MEMORY; }
+#pragma omp parallel for schedule(static) if (nb > LAYOUT_OMP)
         for (int sl = 0; sl < h.nsl; sl++) {
             int k0 = h.sptr[sl], w = h.sptr[sl + 1] - k0;
             for (int l = 0; l < SELLW; l++) {
@@ -1296,6 +1318,7 @@ static int build_bsr(jxamd_solver *s, const jxamd_bsr *A)
         double *v = (double *)calloc(slots * bb * SELLW + 1, sizeof(double));
         double *dinv = (double *)malloc(sizeof(double) * (size_t)nb * bb + 8);
         if (!v || !dinv) { free(v); free(dinv); hsell_free(&h); return JXAMD_ERROR_MEMORY; }
+#pragma omp parallel for schedule(static) if (nb > LAYOUT_OMP)
         for (int sl = 0; sl < h.nsl; sl++) {
             int k0 = h.sptr[sl], w = h.sptr[sl + 1] - k0;
             for (int l = 0; l < SELLW; l++) {
@@ -1309,6 +1332,7 @@ static int build_bsr(jxamd_solver *s, const jxamd_bsr *A)
                 }
             }
         }
+#pragma omp parallel for schedule(static) if (nb > LAYOUT_OMP)
         for (int i = 0; i < nb; i++) block_solve_matrix(A->a + (size_t)A->ia[i] * bb, b, dinv + (size_t)i * bb);
         /* one partitioned sweep (k_bhgs_part) reads the SpMV layout (every
          * stored block but the identity diagonal ones, with their column
@@ -1327,6 +1351,7 @@ static int build_bsr(jxamd_solver *s, const jxamd_bsr *A)
             if (s->prm.stage2_chunk > 0) {
                 const int parts = (nb + s->prm.stage2_chunk - 1) / s->prm.stage2_chunk, size = nb / parts;
                 const int rest = nb - size * parts, big = rest * (size + 1);
+#pragma omp parallel for schedule(static) reduction(+ : whole) if (nb > LAYOUT_OMP)
                 for (int i = 0; i < nb; i++) {
                     const int ns = i < big ? i / (size + 1) * (size + 1) : big + (i - big) / size * size;
                     for (int k = A->ia[i] + 1; k < A->ia[i + 1]; k++) whole += A->ja[k] >= ns && A->ja[k] < i;
@@ -1340,6 +1365,7 @@ static int build_bsr(jxamd_solver *s, const jxamd_bsr *A)
             if (!inv) { free(v); free(dinv); hsell_free(&h); hsched_free(&sc); return JXAMD_ERROR_MEMORY; }
             for (int q = 0; q < npos; q++)
                 if (perm[q] >= 0) inv[perm[q]] = q;
+#pragma omp parallel for schedule(static) if (nb > LAYOUT_OMP)
             for (int sl = 0; sl < h.nsl; sl++)
                 for (int k = h.sptr[sl]; k < h.sptr[sl + 1]; k++)
                     for (int l = 0; l < SELLW; l++) {
