@@ -335,8 +335,10 @@ __device__ __forceinline__ void wave_sync()
 template <int B, int T>
 __global__ void __launch_bounds__(256) k_decouple_apply(int nb, const int *__restrict__ ia, double *a, double *rhs,
                                                         int thermal, const double *__restrict__ coef, int pidx,
-                                                        double *__restrict__ p_a)
+                                                        double *__restrict__ p_a, const int *__restrict__ stop)
 {
+    if (stop && *stop) return; // the coefficients could not be formed: nothing is modified
+
     constexpr int BB = B * B;
     constexpr int WPB = 4; // wavefronts per workgroup
     __shared__ double sv[WPB][WAVE_DC * BB];
@@ -422,6 +424,98 @@ __global__ void __launch_bounds__(256) k_decouple_apply(int nb, const int *__res
     }
 }
 
+// values next to each other, loaded at once from any aligned element
+struct __attribute__((packed, aligned(4))) i32x4 { int v[4]; };
+struct __attribute__((packed, aligned(4))) i32x2 { int v[2]; };
+struct __attribute__((packed, aligned(8))) f64x2 { double v[2]; };
+
+// Column sums of column c over the transpose entries of row c, at most D
+// blocks (nnz >= 4 blocks in all): the row's columns sorted in registers, then
+// the transpose entries of all of them searched together, four entries of each
+// row at a time, then the sum in ascending row order.  False: a transpose
+// entry is missing.  Every lane reads other lines, so a load takes a cycle per
+// lane whatever its width, and these cycles bound the kernel: four indices
+// or two values a load, windows moved back where they would pass the
+// arrays' end.  57x63x41, 3x3: 44 us with loops over the row's length (the
+// arrays in scratch memory), 54 with one value a load, 32 now.
+template <int B, int D>
+__device__ __forceinline__ bool column_sums(int nb, int nnz, int c, const int *__restrict__ ia,
+                                            const int *__restrict__ ja, const double *__restrict__ a,
+                                            double (&ac)[B * B])
+{
+    constexpr int BB = B * B, NS = B == 4 ? 2 : 4; // blocks loaded at once
+    const int cb = ia[c], ce = ia[c + 1];
+    bool ok = true;
+    int cols[D], rb[D], re[D], pos[D];
+#pragma unroll
+    for (int n = 0; n < D; n += 4) {
+        const int s0 = min(cb + n, nnz - 4);
+        const i32x4 w = *reinterpret_cast<const i32x4 *>(ja + s0);
+#pragma unroll
+        for (int h = 0; h < 4; h++) cols[n + h] = s0 + h >= cb + n && s0 + h < ce ? w.v[h] : 0x7fffffff;
+    }
+#pragma unroll
+    for (int pass = 0; pass < D; pass++)
+#pragma unroll
+        for (int n = pass & 1; n + 1 < D; n += 2) {
+            const int lo = min(cols[n], cols[n + 1]), hi = max(cols[n], cols[n + 1]);
+            cols[n] = lo;
+            cols[n + 1] = hi;
+        }
+    int maxlen = 0;
+    bool on[D]; // a column, not seen before
+#pragma unroll
+    for (int n = 0; n < D; n++) {
+        on[n] = cols[n] != 0x7fffffff && (n == 0 || cols[n] != cols[n - 1]);
+        if (on[n] && (cols[n] < 0 || cols[n] >= nb)) ok = false;
+        const i32x2 w = *reinterpret_cast<const i32x2 *>(ia + (on[n] && ok ? cols[n] : c));
+        rb[n] = w.v[0];
+        re[n] = w.v[1];
+        pos[n] = -1;
+    }
+#pragma unroll
+    for (int n = 0; n < D; n++)
+        if (on[n]) maxlen = max(maxlen, re[n] - rb[n]);
+    for (int t = 0; t < maxlen && ok; t += 4) {
+        i32x4 q[D];
+#pragma unroll
+        for (int n = 0; n < D; n++)
+            if (on[n]) q[n] = *reinterpret_cast<const i32x4 *>(ja + min(rb[n] + t, nnz - 4));
+#pragma unroll
+        for (int n = 0; n < D; n++)
+#pragma unroll
+            for (int h = 0; h < 4; h++) {
+                const int k = min(rb[n] + t, nnz - 4) + h;
+                if (on[n] && pos[n] < 0 && k >= rb[n] && k < re[n] && q[n].v[h] == c) pos[n] = k;
+            }
+    }
+#pragma unroll
+    for (int n = 0; n < D; n++)
+        if (on[n] && pos[n] < 0) ok = false;
+#pragma unroll
+    for (int n0 = 0; n0 < D; n0 += NS) {
+        double v[NS][BB];
+#pragma unroll
+        for (int n = 0; n < NS; n++) {
+            if (pos[n0 + n] < 0) continue;
+            const double *blk = a + (size_t)pos[n0 + n] * BB;
+#pragma unroll
+            for (int e = 0; e + 1 < BB; e += 2) {
+                const f64x2 w = *reinterpret_cast<const f64x2 *>(blk + e);
+                v[n][e] = w.v[0];
+                v[n][e + 1] = w.v[1];
+            }
+            if (BB & 1) v[n][BB - 1] = blk[BB - 1];
+        }
+#pragma unroll
+        for (int n = 0; n < NS; n++)
+            if (pos[n0 + n] >= 0)
+#pragma unroll
+                for (int e = 0; e < BB; e++) ac[e] += v[n][e];
+    }
+    return ok;
+}
+
 // True-IMPES coefficients of row c from the column sums Ac_c = sum_i A_ic
 // (rows in ascending order, from zero; jxf_bsr_decoup.c:727-746, 917-935):
 // with a structurally symmetric pattern the rows holding column c are the
@@ -432,56 +526,18 @@ __global__ void __launch_bounds__(256) k_timpes_coef(int nb, const int *__restri
                                                      int *err)
 {
     constexpr int BB = B * B;
+    const int nnz = ia[nb];
     for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < nb; c += gridDim.x * blockDim.x) {
         double ac[BB];
 #pragma unroll
         for (int e = 0; e < BB; e++) ac[e] = 0.0;
         const int cb = ia[c], ce = ia[c + 1];
         bool ok = true;
-        if (ce - cb <= TC_MAXD) {
-            // short rows: the row's distinct columns sorted in registers, then
-            // every transpose search advanced one entry per step for all
-            // columns at once (independent loads), then the sum in ascending
-            // row order
-            int cols[TC_MAXD], rb[TC_MAXD], re[TC_MAXD], pos[TC_MAXD];
-            const int deg = ce - cb;
-#pragma unroll
-            for (int n = 0; n < TC_MAXD; n++) cols[n] = n < deg ? ja[cb + n] : 0x7fffffff;
-            // insertion sort, repeated columns dropped
-#pragma unroll
-            for (int n = 1; n < TC_MAXD; n++) {
-                const int v = cols[n];
-                int q = n - 1;
-                while (q >= 0 && cols[q] > v) {
-                    cols[q + 1] = cols[q];
-                    q--;
-                }
-                cols[q + 1] = v;
-            }
-            int nd = 0;
-#pragma unroll
-            for (int n = 0; n < TC_MAXD; n++)
-                if (cols[n] != 0x7fffffff && (nd == 0 || cols[n] != cols[nd - 1])) cols[nd++] = cols[n];
-            int maxlen = 0;
-            for (int n = 0; n < nd; n++) {
-                if (cols[n] < 0 || cols[n] >= nb) ok = false;
-                rb[n] = ok ? ia[cols[n]] : 0;
-                re[n] = ok ? ia[cols[n] + 1] : 0;
-                pos[n] = -1;
-                if (re[n] - rb[n] > maxlen) maxlen = re[n] - rb[n];
-            }
-            for (int t = 0; t < maxlen && ok; t++)
-                for (int n = 0; n < nd; n++)
-                    if (pos[n] < 0 && rb[n] + t < re[n] && ja[rb[n] + t] == c) pos[n] = rb[n] + t;
-            for (int n = 0; n < nd && ok; n++) {
-                if (pos[n] < 0) { ok = false; break; }
-                const double *blk = a + (size_t)pos[n] * BB;
-#pragma unroll
-                for (int e = 0; e < BB; e++) ac[e] += blk[e];
-            }
-        }
+        const bool any = ce - cb > TC_MAXD || nnz < 4;
+        if (!any && ce - cb <= 8) ok = column_sums<B, 8>(nb, nnz, c, ia, ja, a, ac);
+        else if (!any) ok = column_sums<B, TC_MAXD>(nb, nnz, c, ia, ja, a, ac);
         int prev = -1;
-        for (int n = 0; ce - cb > TC_MAXD && n < ce - cb && ok; n++) {
+        for (int n = 0; any && n < ce - cb && ok; n++) {
             // the next row in ascending order among row c's columns
             int i = 0x7fffffff;
             for (int k = cb; k < ce; k++) {
@@ -531,6 +587,8 @@ __global__ void __launch_bounds__(256) k_timpes_coef(int nb, const int *__restri
     }
 }
 
+__global__ void k_clear(int *p) { *p = 0; }
+
 __global__ void k_pressure_values(long long nnzb, int bb, int pos, const double *__restrict__ a,
                                   double *__restrict__ p_a)
 {
@@ -541,16 +599,16 @@ __global__ void k_pressure_values(long long nnzb, int bb, int pos, const double 
 
 template <int B>
 int launch_apply(int type, int nb, const int *ia, double *a, double *rhs, int thermal, const double *coef, int pidx,
-                 double *p_a, hipStream_t st)
+                 double *p_a, const int *stop, hipStream_t st)
 {
     const int grid = (nb + DC_ROWS - 1) / DC_ROWS;
     switch (type) {
-    case JXAMD_DECOUP_ABF: k_decouple_apply<B, JXAMD_DECOUP_ABF><<<grid, DC_ROWS, 0, st>>>(nb, ia, a, rhs, thermal, coef, pidx, p_a); break;
-    case JXAMD_DECOUP_ANL: k_decouple_apply<B, JXAMD_DECOUP_ANL><<<grid, DC_ROWS, 0, st>>>(nb, ia, a, rhs, thermal, coef, pidx, p_a); break;
-    case JXAMD_DECOUP_SEM: k_decouple_apply<B, JXAMD_DECOUP_SEM><<<grid, DC_ROWS, 0, st>>>(nb, ia, a, rhs, thermal, coef, pidx, p_a); break;
-    case JXAMD_DECOUP_QI: k_decouple_apply<B, JXAMD_DECOUP_QI><<<grid, DC_ROWS, 0, st>>>(nb, ia, a, rhs, thermal, coef, pidx, p_a); break;
-    case JXAMD_DECOUP_TIMPES: k_decouple_apply<B, JXAMD_DECOUP_TIMPES><<<grid, DC_ROWS, 0, st>>>(nb, ia, a, rhs, thermal, coef, pidx, p_a); break;
-    default: k_decouple_apply<B, JXAMD_DECOUP_TIMPES2><<<grid, DC_ROWS, 0, st>>>(nb, ia, a, rhs, thermal, coef, pidx, p_a); break;
+    case JXAMD_DECOUP_ABF: k_decouple_apply<B, JXAMD_DECOUP_ABF><<<grid, DC_ROWS, 0, st>>>(nb, ia, a, rhs, thermal, coef, pidx, p_a, stop); break;
+    case JXAMD_DECOUP_ANL: k_decouple_apply<B, JXAMD_DECOUP_ANL><<<grid, DC_ROWS, 0, st>>>(nb, ia, a, rhs, thermal, coef, pidx, p_a, stop); break;
+    case JXAMD_DECOUP_SEM: k_decouple_apply<B, JXAMD_DECOUP_SEM><<<grid, DC_ROWS, 0, st>>>(nb, ia, a, rhs, thermal, coef, pidx, p_a, stop); break;
+    case JXAMD_DECOUP_QI: k_decouple_apply<B, JXAMD_DECOUP_QI><<<grid, DC_ROWS, 0, st>>>(nb, ia, a, rhs, thermal, coef, pidx, p_a, stop); break;
+    case JXAMD_DECOUP_TIMPES: k_decouple_apply<B, JXAMD_DECOUP_TIMPES><<<grid, DC_ROWS, 0, st>>>(nb, ia, a, rhs, thermal, coef, pidx, p_a, stop); break;
+    default: k_decouple_apply<B, JXAMD_DECOUP_TIMPES2><<<grid, DC_ROWS, 0, st>>>(nb, ia, a, rhs, thermal, coef, pidx, p_a, stop); break;
     }
     return dc_chk(hipGetLastError(), "launch");
 }
@@ -596,30 +654,28 @@ int jxamd_bsr_decouple_device(int nb, int b, const int *d_ia, const int *d_ja, d
         if (hipMalloc(&coef, sizeof(double) * (size_t)nb * b + sizeof(int) * 64) != hipSuccess)
             return JXAMD_ERROR_MEMORY;
         err = (int *)(coef + (size_t)nb * b);
-        if (hipMemsetAsync(err, 0, sizeof(int), st) != hipSuccess) e = JXAMD_ERROR_DEVICE;
+        k_clear<<<1, 1, 0, st>>>(err);
         const int second = type == JXAMD_DECOUP_TIMPES2;
-        if (!e) {
-            switch (b) {
-            case 2: e = launch_coef<2>(second, nb, d_ia, d_ja, d_a, coef, err, st); break;
-            case 3: e = launch_coef<3>(second, nb, d_ia, d_ja, d_a, coef, err, st); break;
-            default: e = launch_coef<4>(second, nb, d_ia, d_ja, d_a, coef, err, st); break;
-            }
+        switch (b) {
+        case 2: e = launch_coef<2>(second, nb, d_ia, d_ja, d_a, coef, err, st); break;
+        case 3: e = launch_coef<3>(second, nb, d_ia, d_ja, d_a, coef, err, st); break;
+        default: e = launch_coef<4>(second, nb, d_ia, d_ja, d_a, coef, err, st); break;
         }
-        int herr = 0;
-        if (!e && (hipMemcpyAsync(&herr, err, sizeof(int), hipMemcpyDeviceToHost, st) != hipSuccess ||
-                   hipStreamSynchronize(st) != hipSuccess))
-            e = JXAMD_ERROR_DEVICE;
-        if (!e && herr) e = JXAMD_ERROR_ARG; // not structurally symmetric: nothing modified
     }
     if (!e) {
         switch (b) {
-        case 2: e = launch_apply<2>(type, nb, d_ia, d_a, d_rhs, thermal, coef, pidx, d_p_a, st); break;
-        case 3: e = launch_apply<3>(type, nb, d_ia, d_a, d_rhs, thermal, coef, pidx, d_p_a, st); break;
-        default: e = launch_apply<4>(type, nb, d_ia, d_a, d_rhs, thermal, coef, pidx, d_p_a, st); break;
+        case 2: e = launch_apply<2>(type, nb, d_ia, d_a, d_rhs, thermal, coef, pidx, d_p_a, err, st); break;
+        case 3: e = launch_apply<3>(type, nb, d_ia, d_a, d_rhs, thermal, coef, pidx, d_p_a, err, st); break;
+        default: e = launch_apply<4>(type, nb, d_ia, d_a, d_rhs, thermal, coef, pidx, d_p_a, err, st); break;
         }
     }
+    // the sweep over the blocks looks at err itself, so that the host waits once
+    int herr = 0;
+    if (err && !e && hipMemcpyAsync(&herr, err, sizeof(int), hipMemcpyDeviceToHost, st) != hipSuccess)
+        e = JXAMD_ERROR_DEVICE;
     const int es = dc_chk(hipStreamSynchronize(st), "synchronise");
     if (es && !e) e = es;
+    if (!e && herr) e = JXAMD_ERROR_ARG; // not structurally symmetric: nothing modified
     if (coef && hipFree(coef) != hipSuccess && !e) e = JXAMD_ERROR_DEVICE;
     return e;
 }
