@@ -1141,7 +1141,7 @@ __global__ void __launch_bounds__(256) k_bhgs_part(int nb, int nparts, int cpb, 
 // column pidx of its block; the other values are read for the in-partition
 // lower blocks alone.  Layouts and results as k_bhgs_part.  Measured, with the
 // general kernel and now: 60x220x85 3x3 118 and 66 us (FP64 blocks), 50 and
-// 40 us (FP16); 61x47x53 4x4 FP64 50 and 27 us; 41x97x37 3x3 FP32 18 and 12 us.
+// 40 us (FP16); 61x47x53 4x4 FP64 50 and 19 us; 41x97x37 3x3 FP32 18 and 12 us.
 template <int B, int LMAX, typename V, typename DV, int PU, typename XP>
 __global__ void __launch_bounds__(256) k_bhgs_first(int nb, int nparts, int cpb, const int *__restrict__ sptr,
                                                     const int *__restrict__ pptr, const int *__restrict__ col,
@@ -1152,6 +1152,7 @@ __global__ void __launch_bounds__(256) k_bhgs_first(int nb, int nparts, int cpb,
 {
     constexpr int LST = (LMAX * (LMAX - 1) / 2) * B * B + 1;
     constexpr bool HALF = constexpr_is_half<V>::value; // slot pairs in 32-bit words, as in k_bhgs_part
+    static_assert(PU <= 8 && LMAX <= 8 && PU % 2 == 0, "four bits per slot; whole slot pairs");
     typedef typename lds_block<V>::T LT;
     extern __shared__ __align__(16) unsigned char smraw[];
     double *sm = reinterpret_cast<double *>(smraw);
@@ -1201,17 +1202,25 @@ __global__ void __launch_bounds__(256) k_bhgs_first(int nb, int nparts, int cpb,
                 for (int rr = 0; rr < B; rr++) pc[HALF ? u / 2 : u][rr] = word(k + u < k1 ? k + u : ks, rr * B + pidx);
 #pragma unroll
             for (int u = 0; u < PU; u++) xj[u] = jj[u] == i ? 0.0 : (double)xp[jj[u]];
+            // in-partition lower blocks: a lane's next one each time round, all
+            // values at once, so that a wavefront whose lanes have them in
+            // different slots pays one trip and not one per slot; four bits per
+            // slot hold the row's place in the partition, from 1
+            unsigned low = 0;
 #pragma unroll
-            for (int u = 0; u < PU; u++) {
-                const int j = jj[u];
-                if (j < ns || j >= i) continue; // in-partition lower blocks
-                LT *L = Lb + (size_t)(c - c0) * LST + ((ti * (ti - 1)) / 2 + (j - ns)) * B * B;
+            for (int u = 0; u < PU; u++)
+                if (jj[u] >= ns && jj[u] < i) low |= (unsigned)(jj[u] - ns + 1) << (4 * u);
+            while (low) {
+                const int u = __builtin_ctz(low) / 4, q = (int)(low >> (4 * u) & 15u) - 1;
+                low &= ~(15u << (4 * u));
+                decltype(word(0, 0)) v[B * B];
+#pragma unroll
+                for (int e = 0; e < B * B; e++) v[e] = word(k + u, e);
+                LT *L = Lb + (size_t)(c - c0) * LST + ((ti * (ti - 1)) / 2 + q) * B * B;
 #pragma unroll
                 for (int e = 0; e < B * B; e++) {
-                    double v;
-                    if constexpr (HALF) v = (double)(u & 1 ? __high2float(word(k + u, e)) : __low2float(word(k + u, e)));
-                    else v = (double)word(k + u, e);
-                    L[e] = (LT)(sc * v);
+                    if constexpr (HALF) L[e] = (LT)(sc * (double)((k + u - ks) & 1 ? __high2float(v[e]) : __low2float(v[e])));
+                    else L[e] = (LT)(sc * (double)v[e]);
                 }
             }
 #pragma unroll
@@ -2020,7 +2029,9 @@ __device__ __forceinline__ double block_sum(double v, double *red)
 // flag (bounded by spin_limit polls: an overflow sets err[0] and the step
 // goes on with whatever hval[k] holds; a waiter that gave up can then arrive
 // at the next reduction before the counter is reset, so after such a step
-// the host must clear cnt and flag before the next launch).
+// the host must clear cnt and flag before the next launch).  A vector that one
+// workgroup holds (16 * 1024 entries) needs none of this: 6144 entries, steps
+// of one to six vectors, 21 us with two workgroups and 11 with one.
 #define MGS_BS 1024 // threads per workgroup of k_mgs_coop: few workgroups, few arrivals per reduction
 
 template <int TM>
@@ -2059,57 +2070,70 @@ __global__ void __launch_bounds__(MGS_BS) k_mgs_coop(size_t n, const double *__r
             for (int t = 0; t < TM; t++) acc += wr[t] * wr[t];
         }
         const double b = block_sum(acc, red);
-        const int target = base + k + 1;
-        double *pk = part + (size_t)k * gridDim.x;
-        if (threadIdx.x == 0) {
-            st_coherent(pk + blockIdx.x, b);
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-            __builtin_amdgcn_s_waitcnt(0);
-            const unsigned int prev = __hip_atomic_fetch_add(cnt, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            last = prev == gridDim.x - 1;
-        }
-        __syncthreads();
-        if (last) {
-            // the last workgroup to arrive sums the partials (every thread a
-            // strided share, then the fixed-order block sum) and publishes h_k
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-            double q = 0.0;
-            for (unsigned int i = threadIdx.x; i < gridDim.x; i += blockDim.x) q += ld_coherent(pk + i);
-            const double sum = block_sum(q, red);
+        if (gridDim.x == 1) {
+            // one workgroup has the sum: nothing to count, publish or wait for;
+            // thread 0 stores the column as it goes, its announcement last
             if (threadIdx.x == 0) {
-                st_coherent(hval + k, sum);
-                __hip_atomic_store(cnt, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                st_flag_release(flag, target);
-                hb = sum;
-            }
-            if (k == m && hhost) {
-                // the whole column to pinned host memory (system-scope
-                // stores), then, if hpos >= 0, the sequence number hseq at
-                // hhost[hpos] once every lane's column stores are ordered
-                // before it: the host may poll that word instead of waiting
-                // for the launch to complete
-                for (int q = threadIdx.x; q <= m; q += blockDim.x)
-                    __hip_atomic_store(hhost + q, q == m ? sum : ld_coherent(hval + q), __ATOMIC_RELAXED,
-                                       __HIP_MEMORY_SCOPE_SYSTEM);
-                if (hpos >= 0) {
-                    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "");
-                    __syncthreads();
-                    if (threadIdx.x == 0) __hip_atomic_store(hhost + hpos, hseq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+                st_coherent(hval + k, b);
+                if (hhost) {
+                    __hip_atomic_store(hhost + k, b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+                    if (k == m && hpos >= 0)
+                        __hip_atomic_store(hhost + hpos, hseq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
                 }
             }
-        } else if (threadIdx.x == 0) {
-            int spins = 0;
-            while (!flag_ready(ld_flag(flag), target)) {
-                if (++spins > spin_limit) {
-                    __hip_atomic_store(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    break;
-                }
+        } else {
+            const int target = base + k + 1;
+            double *pk = part + (size_t)k * gridDim.x;
+            if (threadIdx.x == 0) {
+                st_coherent(pk + blockIdx.x, b);
+                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+                __builtin_amdgcn_s_waitcnt(0);
+                const unsigned int prev = __hip_atomic_fetch_add(cnt, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                last = prev == gridDim.x - 1;
             }
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-            hb = ld_coherent(hval + k);
+            __syncthreads();
+            if (last) {
+                // the last workgroup to arrive sums the partials (every thread a
+                // strided share, then the fixed-order block sum) and publishes h_k
+                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+                double q = 0.0;
+                for (unsigned int i = threadIdx.x; i < gridDim.x; i += blockDim.x) q += ld_coherent(pk + i);
+                const double sum = block_sum(q, red);
+                if (threadIdx.x == 0) {
+                    st_coherent(hval + k, sum);
+                    __hip_atomic_store(cnt, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    st_flag_release(flag, target);
+                    hb = sum;
+                }
+                if (k == m && hhost) {
+                    // the whole column to pinned host memory (system-scope
+                    // stores), then, if hpos >= 0, the sequence number hseq at
+                    // hhost[hpos] once every lane's column stores are ordered
+                    // before it: the host may poll that word instead of waiting
+                    // for the launch to complete
+                    for (int q = threadIdx.x; q <= m; q += blockDim.x)
+                        __hip_atomic_store(hhost + q, q == m ? sum : ld_coherent(hval + q), __ATOMIC_RELAXED,
+                                           __HIP_MEMORY_SCOPE_SYSTEM);
+                    if (hpos >= 0) {
+                        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "");
+                        __syncthreads();
+                        if (threadIdx.x == 0) __hip_atomic_store(hhost + hpos, hseq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+                    }
+                }
+            } else if (threadIdx.x == 0) {
+                int spins = 0;
+                while (!flag_ready(ld_flag(flag), target)) {
+                    if (++spins > spin_limit) {
+                        __hip_atomic_store(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                        break;
+                    }
+                }
+                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+                hb = ld_coherent(hval + k);
+            }
+            __syncthreads();
         }
-        __syncthreads();
-        const double h = hb;
+        const double h = gridDim.x == 1 ? b : hb;
         if (k < m) {
 #pragma unroll
             for (int t = 0; t < TM; t++) wr[t] -= h * vr[t];
@@ -2122,7 +2146,7 @@ __global__ void __launch_bounds__(MGS_BS) k_mgs_coop(size_t n, const double *__r
                 if (e < n) w[e] = wr[t] * sc;
             }
         }
-        __syncthreads(); // hb and last are rewritten by the next reduction
+        if (gridDim.x > 1) __syncthreads(); // hb and last are rewritten by the next reduction
     }
 }
 
@@ -2463,28 +2487,30 @@ int jxamd_k_bhgs_part(int b, int vt, int nb, int nparts, const int *sptr, const 
     // FP32 4, FP16 2 (66 -> 52 us against 4: 75 instead of 109 VGPRs, six
     // waves per SIMD instead of four)
     constexpr int PU64 = 6, PU32 = 4, PU16 = 2;
-    constexpr int PUF = 6; // k_bhgs_first: the stencil's off-diagonals at once
+    // k_bhgs_first: the stencil's off-diagonals at once; FP16 four (six: 84
+    // instead of 66 VGPRs, 44.6 us against 40.3 on 60x220x85; two 41.0)
+    constexpr int PUF = 6, PUF16 = 4;
 #define LAUNCH_PART(BS, LM)                                                                                            \
     do {                                                                                                               \
         const int cpb = 256 / LM;                                                                                      \
         const int grid = (nparts + cpb - 1) / cpb;                                                                     \
         const size_t lb = (size_t)cpb * ((LM * (LM - 1) / 2) * BS * BS + 1);                                          \
         const size_t lds = sizeof(double) * 2 * 256 * BS + (vt == JXAMD_T_F64 ? sizeof(double) : sizeof(float)) * lb; \
-        if (vt == JXAMD_T_F64) LAUNCH_PART_V(BS, LM, double, double, PU64);                                           \
-        else if (vt == JXAMD_T_F32) LAUNCH_PART_V(BS, LM, float, float, PU32);                                        \
-        else LAUNCH_PART_V(BS, LM, __half, float, PU16);                                                               \
+        if (vt == JXAMD_T_F64) LAUNCH_PART_V(BS, LM, double, double, PU64, PUF);                                      \
+        else if (vt == JXAMD_T_F32) LAUNCH_PART_V(BS, LM, float, float, PU32, PUF);                                   \
+        else LAUNCH_PART_V(BS, LM, __half, float, PU16, PUF16);                                                        \
     } while (0)
-#define LAUNCH_PART_V(BS, LM, VT, DT, PU)                                                                              \
+#define LAUNCH_PART_V(BS, LM, VT, DT, PU, PF)                                                                          \
     do {                                                                                                               \
         if (xo)                                                                                                        \
             k_bhgs_part<BS, LM, VT, DT, PU><<<grid, 256, lds, st>>>(nb, nparts, cpb, sptr, pptr, col, (const VT *)val, \
                                                                     rsc, (const DT *)dinv, rhs, xo, xn, w, omega);     \
         else if (xp_f32)                                                                                               \
-            k_bhgs_first<BS, LM, VT, DT, PUF, float><<<grid, 256, lds, st>>>(                                          \
+            k_bhgs_first<BS, LM, VT, DT, PF, float><<<grid, 256, lds, st>>>(                                          \
                 nb, nparts, cpb, sptr, pptr, col, (const VT *)val, rsc, (const DT *)dinv, rhs, (const float *)xp,      \
                 pidx, xn, w, omega);                                                                                   \
         else                                                                                                           \
-            k_bhgs_first<BS, LM, VT, DT, PUF, double><<<grid, 256, lds, st>>>(                                         \
+            k_bhgs_first<BS, LM, VT, DT, PF, double><<<grid, 256, lds, st>>>(                                         \
                 nb, nparts, cpb, sptr, pptr, col, (const VT *)val, rsc, (const DT *)dinv, rhs, (const double *)xp,     \
                 pidx, xn, w, omega);                                                                                   \
     } while (0)
@@ -2822,6 +2848,9 @@ int jxamd_mgs_coop_plan(size_t n, int coop_launch, int *grid, int *tm)
     const void *fn[3] = {(const void *)k_mgs_coop<4>, (const void *)k_mgs_coop<8>, (const void *)k_mgs_coop<16>};
     const int tms[3] = {4, 8, 16};
     for (int q = 0; q < 3; q++) {
+        // one workgroup where it covers n: a reduction across workgroups costs
+        // some 5 us, more than one CU takes to read 16384 entries
+        if (n <= 16 * MGS_BS && n > MGS_BS * (size_t)tms[q]) continue;
         int per = 0;
         if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, fn[q], MGS_BS, 0) != hipSuccess)
             return JXAMD_ERROR_DEVICE;
