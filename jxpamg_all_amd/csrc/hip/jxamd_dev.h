@@ -110,7 +110,9 @@ int jxamd_k_gs_lds(int G, int U, int waves, int xt, int n, const jxamd_lds_sweep
                    void *work, void *stream) __attribute__((weak));
 /* stage 2: x^(-1) into slice order, then K fused sweeps (columns of the
  * layout are positions, ~pos for lower neighbours; xs holds K slice-ordered
- * vectors of xstride doubles; the last sweep also writes xout in row order) */
+ * vectors of xstride doubles; the last sweep also writes xout in row order).
+ * sflag: gate flags, as in the other sync-free launches; dall, the slices whose
+ * earlier sweep a slice reads, orders vorder and is not read on the device */
 int jxamd_k_bhgs_gather(int npos, int b, const int *perm, const double *x0, const double *xp, int pidx, double *out,
                         void *stream);
 int jxamd_k_bhgs_multi(int b, int nsl, int K, const int *vorder, const int *perm, const int *sptr, const int *col,

@@ -2488,7 +2488,7 @@ int jxamd_k_bhgs_part(int b, int vt, int nb, int nparts, const int *sptr, const 
     // waves per SIMD instead of four)
     constexpr int PU64 = 6, PU32 = 4, PU16 = 2;
     // k_bhgs_first: the stencil's off-diagonals at once; FP16 four (six: 84
-    // instead of 66 VGPRs, 44.6 us against 40.3 on 60x220x85; two 41.0)
+    // instead of 71 VGPRs, 44.6 us against 40.3 on 60x220x85; two 41.0)
     constexpr int PUF = 6, PUF16 = 4;
 #define LAUNCH_PART(BS, LM)                                                                                            \
     do {                                                                                                               \
