@@ -554,14 +554,20 @@ template <int U, int G, int ST, typename V, typename X> struct gs_batch {
     {
         return j[u] >= 0 && j[u] != i && (dir > 0 ? j[u] < i : j[u] > i) == dep;
     }
-    // sum over the couplings that are no dependencies, entry values x
+    // sum over the couplings that are no dependencies, entry values x (a
+    // dependency's own value, which may be infinite, does not meet the zero)
     __device__ __forceinline__ X others(int i, int dir, const X *x) const
     {
         X xv[U], acc = 0;
+        V vv[U];
 #pragma unroll
-        for (int u = 0; u < U; u++) xv[u] = coupled(u, i, dir, false) ? x[j[u]] : (X)0;
+        for (int u = 0; u < U; u++) {
+            const bool use = coupled(u, i, dir, false);
+            xv[u] = use ? x[j[u]] : (X)0;
+            vv[u] = use ? v[u] : (V)0;
+        }
 #pragma unroll
-        for (int u = 0; u < U; u++) acc += (X)cvt(v[u]) * xv[u];
+        for (int u = 0; u < U; u++) acc += (X)cvt(vv[u]) * xv[u];
         return acc;
     }
     // sum over the dependencies, this launch's values x
