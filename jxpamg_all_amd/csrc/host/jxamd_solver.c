@@ -65,6 +65,7 @@ typedef struct {
     int unit_diag;             /* every diagonal block is exactly the identity: the partitioned sweeps skip Dinv */
     double part_bytes, part_bytes32; /* algorithmic bytes of one partitioned sweep (FP64, narrow blocks) */
     double first_less;               /* block values the sweep from the prolongated pressure does not need */
+    double *x0;                      /* the prolongated pressure as a vector, where a block holds Inf or NaN (else NULL) */
 } dbsr;
 
 /* one BILU(0) triangle on the device: level-ordered block SELL of the
@@ -1265,7 +1266,13 @@ static int build_bsr(jxamd_solver *s, const jxamd_bsr *A)
         size_t slots = (size_t)(h.nsl ? h.sptr[h.nsl] : 0);
         double *v = (double *)calloc(slots * bb * SELLW + 1, sizeof(double));
         if (!v) { hsell_free(&h); return JXAMD_ERROR_MEMORY; }
-#pragma omp parallel for schedule(static) if (nb > LAYOUT_OMP)
+        /* the sweep from the prolongated pressure (k_bhgs_first) leaves out
+         * products of block values with zeros: only where all values, as
+         * stored, are finite.  Else the pressure becomes a vector and every
+         * sweep is the general one. */
+        const int f32 = s->prm.stage2_precision == 1;
+        int bad = 0;
+#pragma omp parallel for schedule(static) reduction(| : bad) if (nb > LAYOUT_OMP)
         for (int sl = 0; sl < h.nsl; sl++) {
             int k0 = h.sptr[sl], w = h.sptr[sl + 1] - k0;
             for (int l = 0; l < SELLW; l++) {
@@ -1274,9 +1281,18 @@ static int build_bsr(jxamd_solver *s, const jxamd_bsr *A)
                 int len = A->ia[i + 1] - A->ia[i] - skip;
                 for (int k = 0; k < w && k < len; k++) {
                     const double *blk = A->a + (size_t)(A->ia[i] + skip + k) * bb;
-                    for (int e2 = 0; e2 < bb; e2++) v[((size_t)(k0 + k) * bb + e2) * SELLW + l] = blk[e2];
+                    double big = 0.0; /* NaN once a value is not finite */
+                    for (int e2 = 0; e2 < bb; e2++) {
+                        v[((size_t)(k0 + k) * bb + e2) * SELLW + l] = blk[e2];
+                        big += 0.0 * (f32 ? (double)(float)blk[e2] : blk[e2]);
+                    }
+                    bad |= big != 0.0 && skip + k > 0;
                 }
             }
+        }
+        if (bad && s->prm.stage2_chunk > 0) {
+            const int e2 = jxamd_dev_malloc((void **)&d->x0, sizeof(double) * nb * b);
+            if (e2) { free(v); hsell_free(&h); return e2; }
         }
         d->nsl = h.nsl;
         /* bytes the SpMV reads and writes: the stored blocks (without the
@@ -2265,7 +2281,7 @@ int jxamd_solver_destroy(jxamd_solver *s)
     jxamd_dev_free(d->gval); jxamd_dev_free(d->dinv); jxamd_dev_free(d->flag);
     jxamd_dev_free(d->gdep_ptr); jxamd_dev_free(d->gdep_list);
     jxamd_dev_free(d->gall_ptr); jxamd_dev_free(d->gall_list); jxamd_dev_free(d->gvorder); jxamd_dev_free(d->xs);
-    jxamd_dev_free(d->val32); jxamd_dev_free(d->dinv32); jxamd_dev_free(d->rsc16); jxamd_dev_free(d->pptr16);
+    jxamd_dev_free(d->x0); jxamd_dev_free(d->val32); jxamd_dev_free(d->dinv32); jxamd_dev_free(d->rsc16); jxamd_dev_free(d->pptr16);
     for (int l = 0; l < JXAMD_MAX_LEVELS; l++) {
         dsell_free(&s->Ares[l]); dsell_free(&s->Gf[l]); dsell_free(&s->Gb[l]); dsell_free(&s->Gc[l]);
         for (int d = 0; d < 2; d++) {
@@ -2585,7 +2601,7 @@ static int cpr_apply(jxamd_solver *s, const double *r, double *x)
     const int m = s->prm.stage2_maxit;
     /* the partitioned sweeps read an FP32 stage-1 result directly */
     const int xp_f32 = s->xt != JXAMD_T_F64 && s->prm.stage1_maxit > 0 && m > 0 && s->prm.stage2_chunk > 0 &&
-                       s->prm.stage2_solver_type == 2;
+                       s->prm.stage2_solver_type == 2 && !s->A.x0;
     double *xp = (double *)s->U[0];
     if (s->xt != JXAMD_T_F64) {
         xp = s->up64;
@@ -2600,7 +2616,8 @@ static int cpr_apply(jxamd_solver *s, const double *r, double *x)
         dbsr *d = &s->A;
         const int parts = (s->nb + s->prm.stage2_chunk - 1) / s->prm.stage2_chunk;
         double *dst = (m % 2 == 1) ? x : s->xtmp;
-        const double *src = NULL;
+        const double *src = d->x0;
+        if (src) CK(jxamd_k_prolong(s->nb, b, pi, xp, d->x0, s->stream));
         for (int it = 0; it < m; it++) {
             int pq = prof_begin(s);
             const int nar = s->prm.stage2_precision; /* 0 FP64, 1 FP32, 2 FP16 blocks */

@@ -9,6 +9,7 @@ import jxpamg_all_amd as jx
 from oracle.cpu_ref import Oracle
 from tests.test_gpu_lds_sweep import level
 from tests.test_gpu_rowgroup import dev, host, trivial_bsr
+from tests.test_gpu_syncfree import block_system
 
 pytestmark = pytest.mark.gpu
 
@@ -41,3 +42,50 @@ def test_exact_sweep_infinite_coupling(n, rowlen, symmetric, prec, upper):
         want = kinds(Oracle(A, H).relax6(0, f, u0))
     assert 0 < np.count_nonzero(want) and np.array_equal(kinds(host(d_u)), want)
     s.close()
+
+
+def faulty_blocks(nb, b, rowlen, pidx, value, where, chunk):
+    """a system with one such value outside column pidx of a block that
+    couples two partitions (where 0), or lies above (1) or below (2) the
+    diagonal inside one; and the row"""
+    A = block_system(nb, b, rowlen, nb + b)
+    T = -(-nb // chunk)
+    part = np.repeat(np.arange(T), [len(p) for p in np.array_split(np.arange(nb), T)])
+    rows = np.repeat(np.arange(nb), np.diff(A.ia))
+    inside = part[rows] == part[A.ja]
+    at = np.nonzero([~inside, inside & (A.ja > rows), inside & (A.ja < rows)][where])[0]
+    k = int(at[len(at) // 2])
+    A.a.reshape(-1, b, b)[k, 0, (pidx + 1) % b] = value
+    return A, int(rows[k])
+
+
+@pytest.mark.parametrize("b", [2, 3, 4])
+@pytest.mark.parametrize("value", [np.inf, np.nan, 1e300])
+@pytest.mark.parametrize("prec,s2p", [(0, 0), (1, 1), (0, 1), (1, 2)])
+def test_first_stage2_sweep_nonfinite_block(b, value, prec, s2p):
+    """the sweep from the prolongated pressure, whose other unknowns are zeros"""
+    nb, chunk = 700, 4
+    for where in range(3):
+        for pidx in (0, b - 1):
+            A, row = faulty_blocks(nb, b, 7, pidx, value, where, chunk)
+            H = jx.amg_setup(*jx.extract_pressure(A, pidx))
+            s = jx.Solver(A, H, jx.default_params(relax_chunk=4, stage2_chunk=chunk, stage2_maxit=1,
+                                                  pressure_index=pidx, precond_precision=prec, stage2_precision=s2p))
+            r = np.random.default_rng(b).standard_normal(A.n)
+            x = dev(np.zeros(A.n))
+            print(f"[gpu] first sweep b {b} value {value} where {where} pidx {pidx} prec {prec} blocks {s2p}", flush=True)
+            s.precond(dev(r).data_ptr(), x.data_ptr())
+            got = kinds(host(x)).reshape(nb, b)
+            s.close()
+            if value == 1e300 and s2p != 1:
+                # finite in FP64; an FP16 row is scaled by its largest value (overflowed scale: only the row's finiteness goes)
+                assert s2p == 2 or not got.any()
+                continue
+            # the value times a zero (below the diagonal: times a new value) in the row, whose
+            # inverted diagonal block spreads it over the row's unknowns, then the partition's later rows
+            assert np.all(got[row] != 0) and (where == 2 or np.all(got[row] == 2))
+            keep = np.ones(nb, bool)
+            T = -(-nb // chunk)
+            p = [q for q in np.array_split(np.arange(nb), T) if row in q][0]
+            keep[p[p >= row]] = False
+            assert not got[keep].any()
