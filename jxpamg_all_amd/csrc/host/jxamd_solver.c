@@ -1975,7 +1975,8 @@ static int build_lds(jxamd_solver *s, int l, const jxamd_csr *A)
 /* The couplings inside the chunks of level l (T chunks) for relax-6 calls from
  * a zero guess (jxamd_k_gs_chunk_zero), where they are at most half of the
  * stored entries: blocks of L rows hold L - 1 values per row against a mean
- * row's entries and their columns. */
+ * row's entries and their columns.  All of them, as stored, must be finite: the
+ * kernel leaves out products with the zeros of the guess. */
 static int build_chunk_zero(jxamd_solver *s, int l, const jxamd_csr *A, int T)
 {
     const int n = A->n, longest = jxamd_gs_chunk_lds_rows(n, T);
@@ -1986,7 +1987,9 @@ static int build_chunk_zero(jxamd_solver *s, int l, const jxamd_csr *A, int T)
     const size_t nv = (size_t)((T + SELLW - 1) / SELLW) * NE * SELLW;
     double *v = (double *)calloc(nv, sizeof(double));
     if (!v) return JXAMD_ERROR_MEMORY;
-#pragma omp parallel for schedule(static) if (n > 20000)
+    const int f32 = s->xt != JXAMD_T_F64;
+    int bad = 0;
+#pragma omp parallel for schedule(static) reduction(| : bad) if (n > LAYOUT_OMP)
     for (int c = 0; c < T; c++) {
         const int ns = c < rest ? c * (size + 1) : c * size + rest, len = c < rest ? size + 1 : size;
         double *vc = v + (size_t)(c / SELLW) * NE * SELLW + c % SELLW;
@@ -1994,9 +1997,12 @@ static int build_chunk_zero(jxamd_solver *s, int l, const jxamd_csr *A, int T)
             for (int k = A->ia[ns + t] + 1; k < A->ia[ns + t + 1]; k++) {
                 const int q = A->ja[k] - ns;
                 if (q < 0 || q >= len || q == t) continue;
-                vc[(size_t)(t * (L - 1) + (q < t ? q : q - 1)) * SELLW] += A->a[k];
+                double *o = &vc[(size_t)(t * (L - 1) + (q < t ? q : q - 1)) * SELLW];
+                *o += A->a[k];
+                bad |= !isfinite(f32 ? (float)*o : *o) || !isfinite(f32 ? (float)A->a[k] : A->a[k]);
             }
     }
+    if (bad) { free(v); return 0; }
     int e = upload_real(&s->Gz[l], v, nv, s->xt, s->stream);
     const int e2 = jxamd_stream_sync(s->stream);
     free(v);

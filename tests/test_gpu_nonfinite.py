@@ -89,3 +89,29 @@ def test_first_stage2_sweep_nonfinite_block(b, value, prec, s2p):
             p = [q for q in np.array_split(np.arange(nb), T) if row in q][0]
             keep[p[p >= row]] = False
             assert not got[keep].any()
+
+
+@pytest.mark.parametrize("value", [-np.inf, np.nan, 1e300])
+@pytest.mark.parametrize("rowlen", [6, 40])
+@pytest.mark.parametrize("prec", [0, 1])
+def test_chunked_zero_guess_nonfinite_coupling(value, rowlen, prec):
+    """a chunk's own coupling meets the zeros of the guess: the chunk is NaN, the others are finite"""
+    n, chunk = 2000, 4
+    ia, ja, a = level(n, rowlen, rowlen)
+    rows = np.repeat(np.arange(n), np.diff(ia))
+    at = np.nonzero((ja // chunk == rows // chunk) & (ja > rows))[0]
+    k = int(at[len(at) // 2])
+    a[k] = value
+    H = jx.Hierarchy([(ia, ja, a, n)], [])
+    A = trivial_bsr(n)
+    s = jx.Solver(A, H, jx.default_params(relax_chunk=chunk, precond_precision=prec, stage2_maxit=0))
+    r = np.random.default_rng(rowlen).standard_normal(A.n)
+    x = dev(np.zeros(A.n))
+    print(f"[gpu] zero guess value {value} mean row {len(ja) / n:.1f} precision {prec}", flush=True)
+    s.precond(dev(r).data_ptr(), x.data_ptr())
+    got = kinds(host(x)).reshape(n, 2)[:, 0]
+    want = np.zeros(n, int)
+    if value != 1e300 or prec:
+        want[rows[k] // chunk * chunk:][:chunk] = 2
+    assert np.array_equal(got, want)
+    s.close()
