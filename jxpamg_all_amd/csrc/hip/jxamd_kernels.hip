@@ -2387,14 +2387,20 @@ int jxamd_k_gs_sweep(int vt, int xt, int nsl, const int *perm, const int *sptr, 
     return chk(hipGetLastError());
 }
 
-int jxamd_gs_lds_rows(int xt)
+// bytes of LDS a workgroup can have on this device (0: not known)
+static int lds_limit()
 {
     int dev = 0, lds = 0;
     if (hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess)
         return 0;
+    return lds;
+}
+
+int jxamd_gs_lds_rows(int xt)
+{
     const size_t xsz = xt == JXAMD_T_F64 ? sizeof(double) : sizeof(float);
-    const long rows = (long)(lds / xsz) - 1; // and the padding column
+    const long rows = (long)(lds_limit() / xsz) - 1; // and the padding column
     return (int)(rows > JXAMD_LDS_ROW ? JXAMD_LDS_ROW : (rows < 0 ? 0 : rows));
 }
 
@@ -2406,11 +2412,14 @@ int jxamd_k_gs_lds(int G, int U, int waves, int xt, int n, const jxamd_lds_sweep
     if (waves < 1 || waves > JXAMD_LDS_WAVES(U, xt) || n > jxamd_gs_lds_rows(xt)) return JXAMD_ERROR_ARG;
     if (fw->steps % LDS_P || bw->steps % LDS_P) return JXAMD_ERROR_ARG;
     const size_t lds = ((size_t)n + 1) * (xt == JXAMD_T_F64 ? sizeof(double) : sizeof(float));
+    const int limit = lds_limit();
     hipStream_t st = (hipStream_t)stream;
+    // the limit belongs to the kernel, which other handles launch with other
+    // sizes, on other threads too: always the device's, never this call's size
 #define LAUNCH_GL(GG, UU, XX, TT)                                                                                      \
     do {                                                                                                               \
         auto kern_ = k_gs_lds<GG, UU, JXAMD_LDS_WAVES(UU, TT), XX>;                                                    \
-        if (hipFuncSetAttribute((const void *)kern_, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) !=         \
+        if (hipFuncSetAttribute((const void *)kern_, hipFuncAttributeMaxDynamicSharedMemorySize, limit) !=            \
             hipSuccess)                                                                                                \
             return JXAMD_ERROR_DEVICE;                                                                                 \
         kern_<<<1, waves * WAVE, lds, st>>>(n, *fw, *bw, order, (const XX *)diag, 2 * ncalls, (const XX *)f, fs,       \
