@@ -221,15 +221,18 @@ int rn_scratch(void **out)
 // Work buffers of the entry point that waits for its result: one of RN_SLOTS
 // in the module's own memory for the call's duration (with an allocation and a
 // release per call, and the launch that clears a fresh counter, a call took
-// 5 us longer); a call that finds none free allocates its own.
+// 5 us longer); a call that finds none free allocates its own, and so does one
+// on a stream that is being captured, whose launch might run after the call.
 #define RN_SLOTS 8
 static __device__ __align__(256) unsigned char slots[RN_SLOTS * RN_SCRATCH_BYTES];
 void *rn_slots_dev[RN_MAX_DEVICES];
 unsigned int rn_slots_used[RN_MAX_DEVICES]; // bit k: slot k, under rn_mutex
 
 // a free slot of this device: its number and address, or -1
-int rn_slot_take(int *dev, void **out)
+int rn_slot_take(hipStream_t st, int *dev, void **out)
 {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) return -1;
     if (hipGetDevice(dev) != hipSuccess || *dev < 0 || *dev >= RN_MAX_DEVICES) return -1;
     std::lock_guard<std::mutex> g(rn_mutex);
     if (!rn_slots_dev[*dev]) {
@@ -263,15 +266,18 @@ int jxamd_bsr_residual_norm(int nb, int b, const int *d_ia, const int *d_ja, con
     hipStream_t st = (hipStream_t)stream;
     void *work = nullptr;
     int dev = 0;
-    const int slot = rn_slot_take(&dev, &work);
+    const int slot = rn_slot_take(st, &dev, &work);
     if (slot < 0 && hipMalloc(&work, RN_SCRATCH_BYTES) != hipSuccess) return JXAMD_ERROR_MEMORY;
     // a slot's counter is zero: at first, and again after every finished launch
     e = rn_launch(nb, b, d_ia, d_ja, d_a, d_x, d_b, d_norms, (double *)work,
                   (unsigned int *)((unsigned char *)work + RN_PART_BYTES), slot < 0, st);
     // the launch must finish before its partials are released
-    if (hipStreamSynchronize(st) != hipSuccess && !e) e = JXAMD_ERROR_DEVICE;
+    const bool ended = hipStreamSynchronize(st) == hipSuccess;
+    if (!ended && !e) e = JXAMD_ERROR_DEVICE;
     if (slot >= 0) {
-        if (!e) rn_slot_give(dev, slot); // else the launch may not have run to its end
+        // whatever the launch reported; where the wait failed, it may not have
+        // run to its end and the slot stays out of use
+        if (ended) rn_slot_give(dev, slot);
     } else if (hipFree(work) != hipSuccess && !e) {
         e = JXAMD_ERROR_DEVICE;
     }

@@ -4,7 +4,7 @@
  * launcher asks of the runtime is checked without a GPU: kernels do not run,
  * device memory is host memory, launches are held to the dynamic LDS size the
  * kernel was allowed.  One check per run:
- *   launch lds
+ *   launch lds | slots
  */
 #include <hip/hip_runtime.h>
 #include <cstdio>
@@ -20,9 +20,11 @@ extern "C" {
 
 static const int LDS_LIMIT = 160 * 1024, LDS_DEFAULT = 64 * 1024;
 static int mallocs, launches;
-static hipError_t last;
+static hipError_t last, sync_error, stale; /* stale: another call's error, found by the next hipGetLastError */
+static hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
 static std::map<const void *, int> lds_allowed;
 static std::function<void()> before_launch;
+static void *arg6; /* the launch's seventh argument (the residual norm's work buffer) */
 
 extern "C" {
 hipError_t hipMalloc(void **p, size_t n) { mallocs++; *p = calloc(1, n ? n : 1); return hipSuccess; }
@@ -31,8 +33,8 @@ hipError_t hipGetDevice(int *d) { *d = 0; return hipSuccess; }
 hipError_t hipGetDeviceCount(int *n) { *n = 1; return hipSuccess; }
 hipError_t hipGetLastError(void)
 {
-    const hipError_t e = last;
-    last = hipSuccess;
+    const hipError_t e = last != hipSuccess ? last : stale;
+    last = stale = hipSuccess;
     return e;
 }
 hipError_t hipGetSymbolAddress(void **p, const void *)
@@ -46,7 +48,7 @@ hipError_t hipFuncSetAttribute(const void *f, hipFuncAttribute a, int v)
     if (a == hipFuncAttributeMaxDynamicSharedMemorySize) lds_allowed[f] = v;
     return hipSuccess;
 }
-hipError_t hipLaunchKernel(const void *f, dim3, dim3, void **, size_t shared, hipStream_t)
+hipError_t hipLaunchKernel(const void *f, dim3, dim3 block, void **args, size_t shared, hipStream_t)
 {
     if (before_launch) {
         std::function<void()> once;
@@ -55,11 +57,13 @@ hipError_t hipLaunchKernel(const void *f, dim3, dim3, void **, size_t shared, hi
     }
     const int allowed = lds_allowed.count(f) ? lds_allowed[f] : LDS_DEFAULT;
     if (shared > (size_t)allowed) return last = hipErrorInvalidValue;
+    if (block.x == 256) arg6 = *(void **)args[6]; /* the kernels that clear have one thread, and one argument */
     launches++;
     return hipSuccess;
 }
 hipError_t hipLaunchCooperativeKernel(const void *, dim3, dim3, void **, unsigned int, hipStream_t) { return hipSuccess; }
-hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t) { return sync_error; }
+hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus *s) { *s = capture; return hipSuccess; }
 hipError_t hipStreamCreateWithFlags(hipStream_t *, unsigned int) { return hipSuccess; }
 hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
 hipError_t hipEventCreate(hipEvent_t *) { return hipSuccess; }
@@ -119,9 +123,42 @@ static void check_lds()
     }
 }
 
+static int norm()
+{
+    static int ia[2] = {0, 1}, ja[1];
+    static double a[4], x[2], b[2], o[2];
+    return jxamd_bsr_residual_norm(1, 2, ia, ja, a, x, b, o, nullptr);
+}
+
+/* the residual norm's work buffers in the module: given back whenever no
+ * launch can still use them, whatever the call returns */
+static void check_slots()
+{
+    CHECK(norm() == 0 && mallocs == 0);
+    const void *first = arg6;
+    for (int k = 0; k < 20; k++) {
+        stale = hipErrorInvalidValue; /* of an earlier call: reported, but the launch was made and has ended */
+        CHECK(norm() == JXAMD_ERROR_DEVICE);
+    }
+    CHECK(norm() == 0 && mallocs == 0);
+    /* a stream being captured: the wait is refused, and the call's memory is its own */
+    capture = hipStreamCaptureStatusActive;
+    sync_error = hipErrorStreamCaptureUnsupported;
+    for (int k = 0; k < 20; k++) CHECK(norm() == JXAMD_ERROR_DEVICE && mallocs == k + 1);
+    capture = hipStreamCaptureStatusNone;
+    sync_error = hipSuccess;
+    CHECK(norm() == 0 && mallocs == 20 && arg6 == first);
+    /* a wait that fails: the launch may still run, its buffer is not handed out again */
+    sync_error = hipErrorUnknown;
+    CHECK(norm() == JXAMD_ERROR_DEVICE && arg6 == first);
+    sync_error = hipSuccess;
+    CHECK(norm() == 0 && mallocs == 20 && arg6 != first);
+}
+
 int main(int argc, char **argv)
 {
     if (argc == 2 && !strcmp(argv[1], "lds")) check_lds();
+    else if (argc == 2 && !strcmp(argv[1], "slots")) check_slots();
     else return 2;
     printf("launches %d mallocs %d fails %d\n", launches, mallocs, fails);
     return fails ? 1 : 0;

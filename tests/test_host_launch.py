@@ -33,3 +33,7 @@ def run(exe, what):
 
 def test_lds_limit_is_no_callers_own(launch):
     run(launch, "lds")
+
+
+def test_residual_norm_buffers_come_back(launch):
+    run(launch, "slots")
