@@ -111,15 +111,15 @@ int jxamd_k_gs_lds(int G, int U, int waves, int xt, int n, const jxamd_lds_sweep
 /* stage 2: x^(-1) into slice order, then K fused sweeps (columns of the
  * layout are positions, ~pos for lower neighbours; xs holds K slice-ordered
  * vectors of xstride doubles; the last sweep also writes xout in row order).
- * sflag: gate flags, as in the other sync-free launches; dall, the slices whose
- * earlier sweep a slice reads, orders vorder and is not read on the device */
+ * sflag: gate flags, as in the other sync-free launches; vorder: the K * nsl
+ * (sweep, slice) items in an order in which each follows the items it reads */
 int jxamd_k_bhgs_gather(int npos, int b, const int *perm, const double *x0, const double *xp, int pidx, double *out,
                         void *stream);
 int jxamd_k_bhgs_multi(int b, int nsl, int K, const int *vorder, const int *perm, const int *sptr, const int *col,
                        const double *val, const double *dinv, const double *rhs, const double *xsl0, double *xs,
-                       long long xstride, double *xout, const int *dlo_ptr, const int *dlo_list, const int *dall_ptr,
-                       const int *dall_list, int *sflag, int epoch, double w, double omega,
-                       unsigned long long *ticket, unsigned long long *base, int *err, void *stream);
+                       long long xstride, double *xout, const int *dlo_ptr, const int *dlo_list, int *sflag,
+                       int epoch, double w, double omega, unsigned long long *ticket, unsigned long long *base,
+                       int *err, void *stream);
 /* one stage-2 sweep as on nparts ranks (partitions of at most 8 rows);
  * blocks vt = F64 (dinv F64), F32 (dinv F32) or F16 scaled by rsc per block
  * row (dinv F32), stored two slots per 32-bit word from pair pptr[s] of each

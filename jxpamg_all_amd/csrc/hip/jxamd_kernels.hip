@@ -838,7 +838,7 @@ __global__ void __launch_bounds__(WAVE *MAXW) k_gs_lds(int n, jxamd_lds_sweep fw
 // Work items are virtual slices v = k*nsl + s taken in the order vorder (the
 // identity if nullptr), a topological order of
 //   (k, s) after (k, s') for s' in dlo(s)   (slices of lower neighbours)
-//   (k, s) after (k-1, s'') for s'' in dall(s) (slices of all neighbours, s)
+//   (k, s) after (k-1, s'') for s'' the slices of all neighbours, and s
 // so sweep k+1 starts on a slice as soon as sweep k has passed its
 // neighbourhood: the K sweeps overlap instead of running back to back.
 // Gate flags: sflag[k*nsl + s].  U slots per batch: the stencil's six for
@@ -2462,12 +2462,12 @@ int jxamd_k_bhgs_gather(int npos, int b, const int *perm, const double *x0, cons
 
 int jxamd_k_bhgs_multi(int b, int nsl, int K, const int *vorder, const int *perm, const int *sptr, const int *col,
                        const double *val, const double *dinv, const double *rhs, const double *xsl0, double *xs,
-                       long long xstride, double *xout, const int *dlo_ptr, const int *dlo_list, const int *dall_ptr,
-                       const int *dall_list, int *sflag, int epoch, double w, double omega,
-                       unsigned long long *ticket, unsigned long long *base, int *err, void *stream)
+                       long long xstride, double *xout, const int *dlo_ptr, const int *dlo_list, int *sflag,
+                       int epoch, double w, double omega, unsigned long long *ticket, unsigned long long *base,
+                       int *err, void *stream)
 {
     if (nsl == 0 || K < 1) return 0;
-    if (!xsl0 || !xs || !xout || (K > 1 && (!vorder || !dall_ptr || !dall_list))) return JXAMD_ERROR_ARG;
+    if (!xsl0 || !xs || !xout || (K > 1 && !vorder)) return JXAMD_ERROR_ARG;
     if ((long long)nsl * K > 0x7fffffffLL) return JXAMD_ERROR_ARG;
     const int nvs = nsl * K;
     const int waves = jxamd_sweep_waves(nvs);

@@ -56,7 +56,7 @@ typedef struct {
     /* forward block-HGS order */
     int gnsl, gnpos, K;      /* K: stage-2 sweeps fused into one launch */
     int *gperm, *gsptr, *gcol, *flag, *gdep_ptr, *gdep_list;
-    int *gall_ptr, *gall_list, *gvorder; /* neighbourhood slices, sweep-overlapped order */
+    int *gvorder;              /* sweep-overlapped order */
     double *gval, *dinv, *xs;  /* xs: x^(k) of the K sweeps in slice order, then x^(-1) */
     void *val32, *dinv32;      /* FP32 (stage2_precision 1) or FP16 blocks (2; FP32 dinv) for the partitioned stage 2 */
     float *rsc16;              /* stage2_precision 2: power-of-two scale per block row */
@@ -1414,8 +1414,6 @@ static int build_bsr(jxamd_solver *s, const jxamd_bsr *A)
             int *nptr = NULL, *nlist = NULL, *ord = NULL;
             rc = build_nbhd(nb, A->ia, A->ja, &sc, perm, &nptr, &nlist);
             if (!rc) rc = build_vorder(&sc, nptr, nlist, d->K, &ord);
-            if (!rc) rc = upload_ints(&d->gall_ptr, nptr, (size_t)sc.nsl + 1, s->stream);
-            if (!rc) rc = upload_ints(&d->gall_list, nlist, (size_t)nptr[sc.nsl], s->stream);
             if (!rc) rc = upload_ints(&d->gvorder, ord, (size_t)sc.nsl * d->K, s->stream);
             if (!rc) rc = jxamd_stream_sync(s->stream);
             free(nptr);
@@ -2286,7 +2284,7 @@ int jxamd_solver_destroy(jxamd_solver *s)
     jxamd_dev_free(d->gperm); jxamd_dev_free(d->gsptr); jxamd_dev_free(d->gcol);
     jxamd_dev_free(d->gval); jxamd_dev_free(d->dinv); jxamd_dev_free(d->flag);
     jxamd_dev_free(d->gdep_ptr); jxamd_dev_free(d->gdep_list);
-    jxamd_dev_free(d->gall_ptr); jxamd_dev_free(d->gall_list); jxamd_dev_free(d->gvorder); jxamd_dev_free(d->xs);
+    jxamd_dev_free(d->gvorder); jxamd_dev_free(d->xs);
     jxamd_dev_free(d->x0); jxamd_dev_free(d->val32); jxamd_dev_free(d->dinv32); jxamd_dev_free(d->rsc16); jxamd_dev_free(d->pptr16);
     for (int l = 0; l < JXAMD_MAX_LEVELS; l++) {
         dsell_free(&s->Ares[l]); dsell_free(&s->Gf[l]); dsell_free(&s->Gb[l]); dsell_free(&s->Gc[l]);
@@ -2550,8 +2548,8 @@ static int bhgs_run(jxamd_solver *s, int K, const double *rhs, const double *x0,
     int e = jxamd_k_bhgs_gather(d->gnpos, d->b, d->gperm, x0, xp, s->prm.pressure_index, xsl0, s->stream);
     if (!e)
         e = jxamd_k_bhgs_multi(d->b, d->gnsl, K, K > 1 ? d->gvorder : NULL, d->gperm, d->gsptr, d->gcol, d->gval,
-                               d->dinv, rhs, xsl0, d->xs, xstride, xn, d->gdep_ptr, d->gdep_list, d->gall_ptr,
-                               d->gall_list, d->flag, s->epoch, w, omega, s->ticket, &s->tbase, s->err, s->stream);
+                               d->dinv, rhs, xsl0, d->xs, xstride, xn, d->gdep_ptr, d->gdep_list,
+                               d->flag, s->epoch, w, omega, s->ticket, &s->tbase, s->err, s->stream);
     prof_end(s, pq, JXAMD_PROF_BHGS_SWEEP, K * d->sweep_bytes);
     return e;
 }
