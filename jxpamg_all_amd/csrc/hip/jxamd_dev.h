@@ -98,16 +98,14 @@ typedef struct {
     const void *val;           /* vector h of lane: (rec * U/E + h) * 64 + lane */
     int steps;
 } jxamd_lds_sweep;
-/* rows of vector type xt that fit the device's LDS (0: not available); a
- * device layer without these two leaves them undefined, and the solver then
- * keeps to jxamd_k_gs_sweep */
-int jxamd_gs_lds_rows(int xt) __attribute__((weak));
+/* rows of vector type xt that fit the device's LDS (0: not available) */
+int jxamd_gs_lds_rows(int xt);
 /* ncalls relax-6 calls (forward, then backward sweep) from uo (NULL: zeros)
  * into un; diag: a_ii and 1 / a_ii of place q at 2 q (a_ii = 0: the row keeps
  * its value); work: 2 (n + JXAMD_LDS_PAD) values of type xt */
 int jxamd_k_gs_lds(int G, int U, int waves, int xt, int n, const jxamd_lds_sweep *fw, const jxamd_lds_sweep *bw,
                    const int *order, const void *diag, int ncalls, const void *f, int fs, const void *uo, void *un,
-                   void *work, void *stream) __attribute__((weak));
+                   void *work, void *stream);
 /* stage 2: x^(-1) into slice order, then K fused sweeps (columns of the
  * layout are positions, ~pos for lower neighbours; xs holds K slice-ordered
  * vectors of xstride doubles; the last sweep also writes xout in row order).
@@ -145,10 +143,9 @@ int jxamd_k_gs_chunk(int vt, int xt, int n, int nchunks, const int *wstep, const
                      void *un, void *stream);
 /* the same from a zero guess, on the chunks' own couplings alone (blk: row t to
  * row q of chunk c, q counted without t, at ((c / 64) L (L - 1) + t (L - 1) +
- * q) 64 + c % 64); L = 2, 4 or 8, at least the longest chunk; a device layer
- * may leave it undefined */
+ * q) 64 + c % 64); L = 2, 4 or 8, at least the longest chunk */
 int jxamd_k_gs_chunk_zero(int L, int xt, int n, int nchunks, const void *blk, const void *diag, const void *f, int fs,
-                          void *un, void *stream) __attribute__((weak));
+                          void *un, void *stream);
 /* row-group variants (G = 4, 8, 16 or 32 lanes per row): SpMV and polynomial
  * step over the SELL-G layout (64/G rows per slice; sptr: slot-row offsets
  * per slice), the chunked smoother over plain CSR */

@@ -1922,7 +1922,7 @@ static int lds_build(const jxamd_solver *s, const jxamd_csr *D, int dir, const i
 static int build_lds(jxamd_solver *s, int l, const jxamd_csr *A)
 {
     dlds *g = &s->Gl[l];
-    const int n = A->n, cap = jxamd_gs_lds_rows && jxamd_k_gs_lds ? jxamd_gs_lds_rows(s->xt) : 0;
+    const int n = A->n, cap = jxamd_gs_lds_rows(s->xt);
     if (n < 1 || n > cap || s->vt != s->xt) return 0;
     int *ord = (int *)malloc(sizeof(int) * (size_t)n), *place = (int *)malloc(sizeof(int) * (size_t)n), *start = NULL;
     double *diag = (double *)calloc(2 * ((size_t)n + JXAMD_LDS_PAD), sizeof(double));
@@ -1980,7 +1980,7 @@ static int build_chunk_zero(jxamd_solver *s, int l, const jxamd_csr *A, int T)
     const int n = A->n, longest = jxamd_gs_chunk_lds_rows(n, T);
     int L = 2;
     while (L < longest) L *= 2;
-    if (!jxamd_k_gs_chunk_zero || s->vt != s->xt || L > 8 || 2.0 * (L - 1) * n > (double)A->ia[n]) return 0;
+    if (s->vt != s->xt || L > 8 || 2.0 * (L - 1) * n > (double)A->ia[n]) return 0;
     const int size = n / T, rest = n - size * T, NE = L * (L - 1);
     const size_t nv = (size_t)((T + SELLW - 1) / SELLW) * NE * SELLW;
     double *v = (double *)calloc(nv, sizeof(double));
