@@ -375,7 +375,8 @@ def main():
     if not args.no_extra:
         extra = {}
         # the reference's own one-thread semantics: sequential relax-6 sweeps
-        # (k_gs_sweep) and the one-rank stage 2 (k_bhgs_multi)
+        # (k_gs_sweep; k_gs_lds, all of a visit in one launch, on small levels)
+        # and the one-rank stage 2 (k_bhgs_multi)
         pe = jx.default_params(tol=1e-6, max_iter=100, k_dim=30, relax_chunk=0, stage2_chunk=0,
                                arnoldi_kernel=args.arnoldi_kernel)
         se = jx.Solver(Ad, H, pe)
@@ -386,8 +387,8 @@ def main():
         se.close()
         extra["reference_exact"] = {
             "s": round(t_e, 4), "iterations": st_e.iterations, "true_rel_res": st_e.true_rel_res,
-            "k_gs_sweep_per_level": {f"level {l}": {"launches": v[0], "ms": round(v[1], 3), "GBs": gbs(v)}
-                                     for l, v in lv.items()},
+            "exact_sweeps_per_level": {f"level {l} {'k_gs_lds' if len(H.A[l][0]) <= 20480 else 'k_gs_sweep'}":
+                                       {"launches": v[0], "ms": round(v[1], 3), "GBs": gbs(v)} for l, v in lv.items()},
             "k_bhgs_multi": {"launches": pr["bhgs_sweep"][0], "ms": round(pr["bhgs_sweep"][1], 3),
                              "GBs": gbs(pr["bhgs_sweep"])}}
         log(f"reference-exact (one-thread relax 6, one-rank stage 2): {t_e * 1e3:.1f} ms iters {st_e.iterations}")
@@ -429,8 +430,11 @@ def main():
     prof = s.profile_read()
     levels = s.profile_read_levels()
     s.profile(False)
-    # the first of an application's partitioned sweeps is k_bhgs_first, the
-    # others are k_bhgs_part; the smoother levels' first calls are k_gs_chunk_zero
+    # names joined by " / " are kernels that share a class, their launches,
+    # times and bytes taken together: the first of an application's partitioned
+    # sweeps is k_bhgs_first, the others are k_bhgs_part; a level's first
+    # chunked call, from a zero guess, is k_gs_chunk_zero where its blocks hold
+    # at most half of the level's entries
     single = {"bhgs_sweep": ("k_bhgs_part<3, 4, double, double, 6> / k_bhgs_first" if s2chunk
                              else "k_bhgs_multi<3, 6>"),
               "bsr_spmv": "k_bsr_spmv<3, 8, true>", "mgs": "k_mgs_coop<16>", "coarse_solve": "k_dense_gemv<double>",
@@ -439,15 +443,21 @@ def main():
 
     def smoother_kernel(l):
         ia = H.A[l][0]
-        m = (ia[-1] / (len(ia) - 1)) if len(ia) > 1 else 0.0
-        if not chunk:
-            return "k_gs_sweep<double, double>"
-        if m < 12:
-            return "k_gs_chunk_lds<4, double, double, true>"
+        n = len(ia) - 1
+        m = ia[-1] / n if n > 0 else 0.0
         g = 4
         while g < 32 and g * 8 < m:
             g *= 2
-        return f"k_gs_chunk_grp<4, {g}, double, double>"
+        if not chunk:
+            # one workgroup where the vector fits its LDS, else one lane or a group of lanes per row
+            return "k_gs_lds" if n < 20480 else "k_gs_sweep" if m < 12 else f"k_gs_sweep_grp<{g}>"
+        rows = 2
+        while rows < chunk:
+            rows *= 2
+        zero = " / k_gs_chunk_zero" if rows <= 8 and 2 * (rows - 1) * n <= ia[-1] else ""
+        if m < 12:
+            return "k_gs_chunk_lds<4, double, double, true>" + zero
+        return f"k_gs_chunk_grp<4, {g}, double, double>" + zero
     cands += [(smoother_kernel(l) + f" (level {l})", v) for l, v in levels.items()]
     dom_name, (n_l, ms_l, by_l) = max(cands, key=lambda c: c[1][1])
     per_launch_ms = ms_l / n_l

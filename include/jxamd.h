@@ -409,8 +409,8 @@ enum {
 };
 int jxamd_solver_profile(jxamd_solver *s, int enable); /* enable also clears the counters */
 int jxamd_solver_profile_read(jxamd_solver *s, int kind, long *launches, double *ms, double *bytes);
-/* the smoother launches (JXAMD_PROF_GS_SWEEP) of one level: one kernel per
- * level, so this is a per-kernel figure */
+/* the smoother launches (JXAMD_PROF_GS_SWEEP) of one level: one kernel, or
+ * two where chunked relax-6 calls from a zero guess have one of their own */
 int jxamd_solver_profile_read_level(jxamd_solver *s, int level, long *launches, double *ms, double *bytes);
 /* nonzero when a sync-free wait hit its spin bound since creation or since
  * the last solve that reported it (0 when healthy).  A solve during which a

@@ -84,7 +84,7 @@ typedef struct {
     jxamd_lds_sweep sw[2]; /* forward, backward */
     int *order;
     void *diag, *work;
-    double abytes;         /* algorithmic bytes of one sweep */
+    double abytes[2];      /* algorithmic bytes of one forward and one backward pass */
 } dlds;
 
 /* per-kernel-class device timing (HIP events around each launch) */
@@ -1961,6 +1961,10 @@ static int build_lds(jxamd_solver *s, int l, const jxamd_csr *A)
             const int e2 = jxamd_stream_sync(s->stream);
             if (!e) e = e2;
         }
+        /* a pass: the direction's dependencies with their columns, the rows'
+         * right-hand side (or what is left of it), diagonal and result */
+        for (int d = 0; d < 2; d++)
+            g->abytes[d] = (double)(s->xsz + sizeof(int)) * D[d].ia[n] + 3.0 * (double)s->xsz * n;
         g->G = G;
         g->U = U;
         g->W = e ? 0 : W;
@@ -2086,9 +2090,7 @@ static int build_level_mats(jxamd_solver *s, int l, const jxamd_hierarchy *H, co
         /* forward + backward pass over the matrix, old + new + rhs vectors */
         s->Gc[l].abytes = 2.0 * level_bytes(&s->Gc[l], A->ia[n], n, 0.0) + 3.0 * type_size(s->xt) * n;
     } else if ((l < s->L - 1 || s->L == 1) && s->Gl[l].W) {
-        /* sweep: matrix once + old x + new x + rhs */
-        dsell t = {.vt = s->vt, .xt = s->xt};
-        s->Gl[l].abytes = level_bytes(&t, A->ia[n], n, 3.0);
+        /* its own layout is built: build_lds */
     } else if ((l < s->L - 1 || s->L == 1) && GA > 1) {
         /* long rows: sweep orders with slices of 64/GA rows of one dependency
          * level, each row summed by a group of GA lanes over its plain CSR
@@ -2382,7 +2384,9 @@ static int hsgs_lds(jxamd_solver *s, int l, const void *f, int fs, void *u, int 
     int pq = prof_begin(s);
     CK(jxamd_k_gs_lds(g->G, g->U, g->W, s->xt, s->nlev[l], &g->sw[0], &g->sw[1], g->order, g->diag, ncalls, f, fs,
                       uo_zero ? NULL : u, u, g->work, s->stream));
-    prof_end_level(s, pq, JXAMD_PROF_GS_SWEEP, l, 2.0 * ncalls * g->abytes);
+    /* from a vector, one more pass for the sums over its upper couplings */
+    prof_end_level(s, pq, JXAMD_PROF_GS_SWEEP, l,
+                   ncalls * (g->abytes[0] + g->abytes[1]) + (uo_zero ? 0.0 : g->abytes[1]));
     return 0;
 }
 

@@ -154,7 +154,23 @@ int main(int argc, char **argv)
             jxamd_solver *s = NULL;
             rc = jxamd_solver_create(&s, &B, &H, &p);
             if (!rc) rc = jxamd_cpr_precond_device(s, r, x); /* from a zero guess, f strided in FP64 */
+            if (!rc) rc = jxamd_solver_profile(s, 1);
+            const int e0 = exact;
             if (!rc) rc = jxamd_op_hsgs(s, 0, r, x);         /* from u */
+            if (!rc && exact > e0) {
+                /* the bytes it is priced at: forward, backward, and the sums
+                 * over the upper couplings before */
+                const double xsz = prec ? 4.0 : 8.0;
+                double ms, bytes = 0.0, want = 9.0 * xsz * n;
+                long count = 0;
+                for (int i = 0; i < n; i++)
+                    for (int k = ia[i] + 1; k < ia[i + 1]; k++) want += (ja[k] < i ? 1.0 : 2.0) * (xsz + 4.0);
+                rc = jxamd_solver_profile_read(s, JXAMD_PROF_GS_SWEEP, &count, &ms, &bytes);
+                if (!rc && (count != 1 || bytes != want)) {
+                    fprintf(stderr, "exact sweep priced at %.0f bytes in %ld launches, not %.0f\n", bytes, count, want);
+                    rc = 10;
+                }
+            }
             if (s) jxamd_solver_destroy(s);
         }
     free(ia); free(ja); free(a); free(ref); free(bi); free(bj); free(ba); free(r); free(x);
