@@ -420,8 +420,10 @@ static int build_vorder(const hsched *sc, const int *nb_ptr, const int *nb_list,
 /* rows from which the host lays a matrix out on all cores; below, the threads'
  * start takes as long as the loop.  Creating a solver from a hierarchy, with
  * one core per layout and with sixteen: 60x220x85 1030 and 418 ms, 61x47x53
- * 4x4 220 and 99 ms. */
-#define LAYOUT_OMP 20000
+ * 4x4 220 and 99 ms.  20x25x20 3x3 in chunks: 10.0 ms with 20000 here (more
+ * than with no threads at all, 7.7: a loop that may run on all cores is the
+ * slower one on a single core), 8.6 with 8000, 8.1 with 4000. */
+#define LAYOUT_OMP 4000
 
 /* Scalar SELL-64 on the host.  Rows in the order given by perm (identity if
  * NULL).  offdiag: drop the first (diagonal) entry of every row into diag[].
@@ -1095,12 +1097,12 @@ static int csr_sorted(int n, const int *ia, const int *ja, const double *a, int 
     double *a2 = (double *)malloc(sizeof(double) * (nnz ? nnz : 1));
     if (!j2 || !a2) { free(j2); free(a2); return JXAMD_ERROR_MEMORY; }
     int bad = 0;
-#pragma omp parallel for schedule(static) reduction(| : bad) if (nnz > 100000)
-    for (int b0 = 0; b0 < n; b0 += 1024) {
+#pragma omp parallel for schedule(static) reduction(| : bad) if (nnz > 20000)
+    for (int b0 = 0; b0 < n; b0 += 64) {
         int cap = 0;
         int *tj = NULL;
         double *ta = NULL;
-        for (int i = b0; i < n && i < b0 + 1024; i++) {
+        for (int i = b0; i < n && i < b0 + 64; i++) {
             const int k0 = ia[i], len = ia[i + 1] - k0, f = keep < len ? keep : len, m = len - f;
             memcpy(j2 + k0, ja + k0, sizeof(int) * (size_t)len);
             memcpy(a2 + k0, a + k0, sizeof(double) * (size_t)len);
@@ -1829,26 +1831,33 @@ static int lds_levels(const jxamd_csr *F, const jxamd_csr *B, int *ord, int **os
     return 0;
 }
 
-/* records of the slice at places b .. e: one per G * U entries of its longest row */
-static int lds_records(const jxamd_csr *D, const int *ord, int b, int e, int GU)
+/* the slices of R rows of every level, in the levels' order: len, the entries
+ * of a slice's longest row (at least one), first[l], the number of level l's
+ * first.  A slice takes one record per G * U entries of its longest row. */
+static void lds_slices(const jxamd_csr *D, const int *ord, const int *start, int nl, int R, int *len, int *first)
 {
-    int len = 1;
-    for (; b < e; b++)
-        if (D->ia[ord[b] + 1] - D->ia[ord[b]] > len) len = D->ia[ord[b] + 1] - D->ia[ord[b]];
-    return (len + GU - 1) / GU;
+    int q = 0;
+    for (int l = 0; l < nl; l++) {
+        first[l] = q;
+        for (int b = start[l]; b < start[l + 1]; b += R, q++) {
+            len[q] = 1;
+            for (int t = b; t < b + R && t < start[l + 1]; t++)
+                if (D->ia[ord[t] + 1] - D->ia[ord[t]] > len[q]) len[q] = D->ia[ord[t] + 1] - D->ia[ord[t]];
+        }
+    }
+    first[nl] = q;
 }
 
-/* steps of a direction's schedule: a level's slices of R rows, W at a time, as
- * many steps as the slice with most records has */
-static long lds_steps(const jxamd_csr *D, const int *ord, const int *start, int nl, int G, int U, int W, long *nrec)
+/* steps of a direction's schedule: a level's slices W at a time, as many steps
+ * as the slice with most records has */
+static long lds_steps(const int *len, const int *first, int nl, int GU, int W, long *nrec)
 {
-    const int R = SELLW / G;
     long steps = 0, recs = 1;
     for (int l = 0; l < nl; l++)
-        for (int b = start[l]; b < start[l + 1];) {
+        for (int q = first[l]; q < first[l + 1];) {
             int most = 0;
-            for (int w = 0; w < W && b < start[l + 1]; w++, b += R) {
-                const int ns = lds_records(D, ord, b, b + R < start[l + 1] ? b + R : start[l + 1], G * U);
+            for (int w = 0; w < W && q < first[l + 1]; w++, q++) {
+                const int ns = (len[q] + GU - 1) / GU;
                 recs += ns;
                 if (ns > most) most = ns;
             }
@@ -1858,12 +1867,14 @@ static long lds_steps(const jxamd_csr *D, const int *ord, const int *start, int 
     return steps;
 }
 
-/* the schedule and records of one direction (dependencies D), uploaded */
+/* the schedule and records of one direction (dependencies D, slices len and
+ * first for this G), uploaded */
 static int lds_build(const jxamd_solver *s, const jxamd_csr *D, int dir, const int *ord, const int *place,
-                     const int *start, int nl, int G, int U, int W, jxamd_lds_sweep *o)
+                     const int *start, int nl, const int *len, const int *first, int G, int U, int W,
+                     jxamd_lds_sweep *o)
 {
     const int R = SELLW / G, n = D->n, xsz = (int)s->xsz, E = 16 / xsz;
-    long nrec = 0, steps = lds_steps(D, ord, start, nl, G, U, W, &nrec);
+    long nrec = 0, steps = lds_steps(len, first, nl, G * U, W, &nrec);
     steps = (steps + JXAMD_LDS_DEPTH - 1) / JXAMD_LDS_DEPTH * JXAMD_LDS_DEPTH;
     const size_t recs = (size_t)nrec, places = (size_t)(steps + 2 * JXAMD_LDS_DEPTH) * W;
     int *sched = (int *)calloc(2 * places, sizeof(int));
@@ -1878,16 +1889,17 @@ static int lds_build(const jxamd_solver *s, const jxamd_csr *D, int dir, const i
             for (int b = start[l]; b < end;) {
                 int most = 0;
                 for (int w = 0; w < W && b < end; w++, b += R) {
-                    const int cnt = b + R < end ? R : end - b, ns = lds_records(D, ord, b, b + cnt, G * U);
+                    const int cnt = b + R < end ? R : end - b;
+                    const int ns = (len[first[l] + (b - start[l]) / R] + G * U - 1) / (G * U);
                     if (ns > most) most = ns;
                     for (int h = 0; h < ns; h++, rec++) {
                         int *q = sched + 2 * ((t + h) * W + w);
                         q[0] = b | cnt << 16 | (h > 0 ? JXAMD_LDS_CONT : 0) | (h == ns - 1 ? JXAMD_LDS_LAST : 0);
                         q[1] = (int)rec;
                         for (int r = 0; r < cnt; r++) {
-                            const int i = ord[b + r], k0 = D->ia[i], len = D->ia[i + 1] - k0;
+                            const int i = ord[b + r], k0 = D->ia[i], rlen = D->ia[i + 1] - k0;
                             /* entry pp of the row: record pp / (G U), slot (pp / G) % U, lane pp % G */
-                            for (int pp = h * G * U; pp < len && pp < (h + 1) * G * U; pp++) {
+                            for (int pp = h * G * U; pp < rlen && pp < (h + 1) * G * U; pp++) {
                                 const int u = (pp / G) % U, lane = r * G + pp % G;
                                 col[((rec * (U / 4) + u / 4) * SELLW + lane) * 4 + u % 4] = place[D->ja[k0 + pp]] * xsz;
                                 val[((rec * (U / E) + u / E) * SELLW + lane) * E + u % E] = D->a[k0 + pp];
@@ -1925,8 +1937,14 @@ static int build_lds(jxamd_solver *s, int l, const jxamd_csr *A)
     const int n = A->n, cap = jxamd_gs_lds_rows(s->xt);
     if (n < 1 || n > cap || s->vt != s->xt) return 0;
     int *ord = (int *)malloc(sizeof(int) * (size_t)n), *place = (int *)malloc(sizeof(int) * (size_t)n), *start = NULL;
+    /* slices of a direction: no more than rows; levels: no more than rows */
+    int *len[2], *first[2];
+    for (int d = 0; d < 2; d++) {
+        len[d] = (int *)malloc(sizeof(int) * (size_t)n);
+        first[d] = (int *)malloc(sizeof(int) * ((size_t)n + 1));
+    }
     double *diag = (double *)calloc(2 * ((size_t)n + JXAMD_LDS_PAD), sizeof(double));
-    int nl = 0, e = !ord || !place || !diag ? JXAMD_ERROR_MEMORY : 0;
+    int nl = 0, e = !ord || !place || !diag || !len[0] || !len[1] || !first[0] || !first[1] ? JXAMD_ERROR_MEMORY : 0;
     jxamd_csr D[2];
     memset(D, 0, sizeof(D));
     for (int d = 0; d < 2 && !e; d++) e = lds_deps(A, d ? -1 : 1, &D[d]);
@@ -1934,17 +1952,19 @@ static int build_lds(jxamd_solver *s, int l, const jxamd_csr *A)
     if (!e && nl) {
         double best = 2.0 * 2.3 * nl;
         int G = 0, U = 0, W = 0;
-        for (int g1 = 1; g1 <= 16; g1 *= 2)
+        for (int g1 = 1; g1 <= 16; g1 *= 2) {
+            for (int d = 0; d < 2; d++) lds_slices(&D[d], ord, start, nl, SELLW / g1, len[d], first[d]);
             for (int u1 = 4; u1 <= 8; u1 += 4)
                 for (int w1 = 1; w1 <= JXAMD_LDS_WAVES(u1, s->xt); w1 *= 2) {
                     double c = 0.0;
                     for (int d = 0; d < 2; d++) {
                         long nrec = 0;
-                        const long steps = lds_steps(&D[d], ord, start, nl, g1, u1, w1, &nrec);
+                        const long steps = lds_steps(len[d], first[d], nl, g1 * u1, w1, &nrec);
                         c += (0.16 + (0.017 + 0.0064 * u1) * w1) * (double)steps + 0.0056 * u1 * (double)nrec;
                     }
                     if (c < best) { best = c; G = g1; U = u1; W = w1; }
                 }
+        }
         if (W) {
             for (int q = 0; q < n; q++) {
                 /* the diagonal as the kernel holds it, and its reciprocal */
@@ -1953,8 +1973,10 @@ static int build_lds(jxamd_solver *s, int l, const jxamd_csr *A)
                 diag[2 * q] = di;
                 diag[2 * q + 1] = di != 0.0 ? 1.0 / di : 0.0;
             }
-            for (int d = 0; d < 2 && !e; d++)
-                e = lds_build(s, &D[d], d ? -1 : 1, ord, place, start, nl, G, U, W, &g->sw[d]);
+            for (int d = 0; d < 2 && !e; d++) {
+                lds_slices(&D[d], ord, start, nl, SELLW / G, len[d], first[d]);
+                e = lds_build(s, &D[d], d ? -1 : 1, ord, place, start, nl, len[d], first[d], G, U, W, &g->sw[d]);
+            }
             if (!e) e = upload_ints(&g->order, ord, (size_t)n, s->stream);
             if (!e) e = upload_real(&g->diag, diag, 2 * ((size_t)n + JXAMD_LDS_PAD), s->xt, s->stream);
             if (!e) e = jxamd_dev_malloc(&g->work, 2 * s->xsz * ((size_t)n + JXAMD_LDS_PAD));
@@ -1970,6 +1992,7 @@ static int build_lds(jxamd_solver *s, int l, const jxamd_csr *A)
         g->W = e ? 0 : W;
     }
     free(ord); free(place); free(start); free(diag);
+    for (int d = 0; d < 2; d++) { free(len[d]); free(first[d]); }
     for (int d = 0; d < 2; d++) { free((void *)D[d].ia); free((void *)D[d].ja); free((void *)D[d].a); }
     return e;
 }
@@ -2133,12 +2156,13 @@ static int build_level_mats(jxamd_solver *s, int l, const jxamd_hierarchy *H, co
 static int build_level(jxamd_solver *s, int l, const jxamd_hierarchy *H)
 {
     /* the level's matrix with sorted rows (the diagonal still first) where
-     * row groups read it; the one-lane-per-row layouts keep the given order */
+     * row groups read it (not the coarsest, whose inverse is applied); the
+     * one-lane-per-row layouts keep the given order */
     const jxamd_csr *A = &H->A[l];
     jxamd_csr S = *A;
     int *sj = NULL;
     double *sa = NULL;
-    if (choose_group(A->ia[A->n], A->n) > 1) {
+    if (choose_group(A->ia[A->n], A->n) > 1 && (l < s->L - 1 || s->L == 1)) {
         CK(csr_sorted(A->n, A->ia, A->ja, A->a, 1, &sj, &sa));
         S.ja = sj;
         S.a = sa;
