@@ -1297,9 +1297,10 @@ __global__ void k_bhgs_gather(int npos, int B, const int *__restrict__ perm, con
 // power of two rsc[p] per block row: M_ij = rsc[p] * stored; FP16 elements
 // stored in pairs, slot k's word w at (k * ceil(B*B/2) + w) * 64 + lane), Dinv as DV,
 // vectors and arithmetic double.  A lane loads the column indices and blocks
-// of its first BT_U slots before it waits, so that a level step costs the
-// dependency values' round trip and no more (out is armed when the launch
-// starts).  The subtractions keep the order of the blocks in the row.
+// of its first BT_U slots, and widens the blocks, before it waits, so that a
+// level step costs the dependency values' round trip and no more (out is armed
+// when the launch starts).  The subtractions keep the order of the blocks in
+// the row.
 #define BT_U 4
 template <int B, typename V, typename DV>
 __global__ void __launch_bounds__(256) k_btri(int nsl, const int *__restrict__ perm, const int *__restrict__ sptr,
@@ -1331,7 +1332,14 @@ __global__ void __launch_bounds__(256) k_btri(int nsl, const int *__restrict__ p
         for (int k = k0; k < k1; k += BT_U) {
             int j[BT_U];
             bool use[BT_U];
-            double xc[BT_U][B], m[BT_U][B * B];
+            double xc[BT_U][B];
+            // FP16: elements 2w and 2w + 1 of a block in one 32-bit word (a
+            // zero high half past the last), so the loads are whole words
+            constexpr bool HALF = constexpr_is_half<V>::value;
+            typedef typename std::conditional<HALF, __half2, V>::type W;
+            constexpr int NW = HALF ? (B * B + 1) / 2 : B * B;
+            W st[BT_U][NW];
+            double m[BT_U][B * B];
 #pragma unroll
             for (int u = 0; u < BT_U; u++) {
                 j[u] = k + u < k1 && i >= 0 ? col[(size_t)(k + u) * WAVE + lane] : i;
@@ -1339,25 +1347,22 @@ __global__ void __launch_bounds__(256) k_btri(int nsl, const int *__restrict__ p
             }
 #pragma unroll
             for (int u = 0; u < BT_U; u++) {
-                const size_t ks = k + u < k1 ? k + u : k0;
-                if constexpr (constexpr_is_half<V>::value) {
-                    // FP16: elements 2w and 2w + 1 of a block in one
-                    // 32-bit word (a zero high half past the last), so
-                    // the loads are whole words
-                    constexpr int NW = (B * B + 1) / 2;
-                    const __half2 *vw = reinterpret_cast<const __half2 *>(val) + ks * NW * WAVE + lane;
+                const W *vw = reinterpret_cast<const W *>(val) + (size_t)(k + u < k1 ? k + u : k0) * NW * WAVE + lane;
 #pragma unroll
-                    for (int w = 0; w < NW; w++) {
-                        const __half2 h = vw[w * WAVE];
-                        m[u][2 * w] = (double)__low2float(h);
-                        if (2 * w + 1 < B * B) m[u][2 * w + 1] = (double)__high2float(h);
-                    }
-                } else {
-                    const V *vv = val + ks * B * B * WAVE + lane;
-#pragma unroll
-                    for (int q = 0; q < B * B; q++) m[u][q] = (double)cvt(vv[q * WAVE]);
-                }
+                for (int w = 0; w < NW; w++) st[u][w] = vw[w * WAVE];
             }
+            // widened and scaled before the wait, where the time is free: the
+            // compiler would do it behind, on every level's critical path
+            // (24x40x21 4x4, both triangles, FP16 527 -> 484 us, with a flag
+            // per slice 490; 30x45x40 3x3 FP16 552 -> 512, FP64 524 -> 518)
+#pragma unroll
+            for (int u = 0; u < BT_U; u++)
+#pragma unroll
+                for (int e = 0; e < B * B; e++) {
+                    if constexpr (HALF) m[u][e] = sc * (double)(e & 1 ? __high2float(st[u][e / 2]) : __low2float(st[u][e / 2]));
+                    else m[u][e] = sc * (double)st[u][e];
+                    asm volatile("" : "+v"(m[u][e]));
+                }
             if (k == k0) wait_gate(sflag, gate, epoch);
             read_results<BT_U, B, double>(out, j, use, xc, err);
 #pragma unroll
@@ -1366,7 +1371,7 @@ __global__ void __launch_bounds__(256) k_btri(int nsl, const int *__restrict__ p
 #pragma unroll
                 for (int r = 0; r < B; r++) {
 #pragma unroll
-                    for (int q = 0; q < B; q++) acc[r] -= (sc * m[u][r * B + q]) * xc[u][q];
+                    for (int q = 0; q < B; q++) acc[r] -= m[u][r * B + q] * xc[u][q];
                 }
             }
         }
