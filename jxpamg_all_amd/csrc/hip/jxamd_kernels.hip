@@ -442,7 +442,7 @@ __global__ void __launch_bounds__(256) k_poly_step(int n, const int *__restrict_
 // bounded: a wave that gives up sets err[0] and goes on with the armed NaN,
 // which arithmetic quiets, so the launch still drains.
 // Measured, with a flag per slice and now: a 3x3 BILU(0) triangle of 30x40x25
-// (93 levels) 261 and 214 us; three stage-2 sweeps of 24x40x21, b = 2, 252 and
+// (93 levels) 261 and 208 us; three stage-2 sweeps of 24x40x21, b = 2, 252 and
 // 134 us, of 16x16x8, b = 3, 126 and 75 us; the reference-exact CPR application
 // of 60x220x85 255 and 89 ms.  A level costs 2.1-2.3 us now.
 // ---------------------------------------------------------------------------
@@ -681,9 +681,9 @@ template <int G, typename X> __device__ __forceinline__ X dpp_sum(X v)
 // f and h lie in the rows' order, too: loads by row number take a cycle per
 // lane (336 us instead of 196 for the first level below).
 // Two calls (four sweeps), with a flag-per-slice k_gs_sweep, with full rows
-// in LDS and now: 20160 rows of 7 (83 levels) 1010, 240 and 196 us; 8807 rows
-// of 23 (261 levels) 3340, 609 and 499; 2114 rows of 61 (374 levels) 4520, 456
-// and 430; 2048 rows of 7 (38 levels) 408, 46 and 39.
+// in LDS and now: 20160 rows of 7 (83 levels) 1010, 240 and 199 us; 8807 rows
+// of 23 (261 levels) 3340, 609 and 496; 2114 rows of 61 (374 levels) 4520, 456
+// and 428; 2048 rows of 7 (38 levels) 408, 46 and 39.
 // A step's time is its wavefronts' instructions as much as its latencies,
 // hence 16-byte loads at scalar base + lane offset, columns as LDS byte
 // offsets, and the quotient from the stored reciprocal.
